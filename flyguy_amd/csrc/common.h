@@ -37,16 +37,25 @@ const char* last_error();
 void clear_error();
 
 // XCD-aware tile mapping: the hardware deals workgroups to the 8 XCDs round robin (block i -> XCD i % 8).
-// With T % 8 == 0 each XCD works through its own tiles x, x+8, ... one after another, row blocks inner, so its
-// L2 holds one tile's source slab at a time.  Otherwise tiles are walked in plain order.
+// Each XCD first works through whole tiles of its own, x, x+8, ..., one after another, row blocks inner, so its L2 holds
+// one tile's source slab at a time.  The T % 8 tiles left are cut into 8 slices each (slice j: row blocks j, j+8, ...,
+// an even sample of a plan sorted by length), and XCD x takes T % 8 consecutive slices, so that all XCDs get the same
+// work and each reads at most two of those slabs.  (Walking all tiles in plain order whenever T % 8 != 0 had every XCD
+// read every slab: B=416, 13 tiles, hop 1 / 2 / 3 forward 142 / 255 / 60 us, with the slices 132 / 178 / 41 us.)
+// A slice may be one block short: rb >= RB is a block without work.
+__host__ __device__ inline long long tile_blocks(int RB, int T) {
+    const int r = T & 7;
+    return (long long)(T - r) * RB + 8LL * r * ((RB + 7) / 8);
+}
 __device__ __forceinline__ int tile_of(int bid, int RB, int T, int& rb) {
-    if ((T & 7) == 0) {
-        int x = bid & 7, s = bid >> 3;
+    const int x = bid & 7, s = bid >> 3, whole = (T >> 3) * RB;
+    if (s < whole) {
         rb = s % RB;
         return x + 8 * (s / RB);
     }
-    rb = bid % RB;
-    return bid / RB;
+    const int per = (RB + 7) / 8, i = x * (T & 7) + (s - whole) / per;      // slice i: slice i % 8 of left tile i / 8
+    rb = (i & 7) + 8 * ((s - whole) % per);
+    return (T & ~7) + (i >> 3);
 }
 
 // a compile-time flag as a type (the hop kernels' step bodies take it: Full<true> for a step whose 8 slots are all

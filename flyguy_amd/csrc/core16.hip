@@ -107,6 +107,7 @@ __global__ __launch_bounds__(WG) void k_cfwd16(Plan p, const int2* __restrict__ 
     extern __shared__ __align__(16) unsigned fires[];
     int rb;
     const int tile = tile_of(blockIdx.x, RB, T, rb);
+    if (rb >= RB) return;
     const bool bits = stage_fires(src_fires, fw_ld, tile, fires);     // (only for a tile with silent source rows)
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
@@ -173,6 +174,7 @@ __global__ __launch_bounds__(FWD_LDS_NW * 64) void k_cfwd16_lds(Plan p, const in
     extern __shared__ __align__(16) u32x4 xs16[];         // the tile's slab, src_rows x 8 (16 bytes each)
     int s;
     const int tile = tile_of(blockIdx.x, S, T, s);
+    if (s >= S) return;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63, gi = grp & 7;
     const int w0 = __builtin_amdgcn_readfirstlane(s * FWD_LDS_NW + (int)(threadIdx.x >> 6)), dw = S * FWD_LDS_NW;
     const int n = w0 < p.nwave ? (p.nwave - 1 - w0) / dw + 1 : 0;
@@ -428,6 +430,7 @@ __global__ __launch_bounds__(WG) void k_cbwd16(Plan p, const int2* __restrict__ 
     __shared__ __align__(16) int2 slots[WG / LPR][LPR];
     int rb;
     const int tile = tile_of(blockIdx.x, RB, T, rb);
+    if (rb >= RB) return;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
@@ -491,6 +494,7 @@ __global__ __launch_bounds__(WG) void k_cbwd16x2(Plan p, const int2* __restrict_
     __shared__ __align__(16) int2 slots[WG / LPR][LPR];
     int rb;
     const int pr = tile_of(blockIdx.x, RB, (T + 1) / 2, rb);
+    if (rb >= RB) return;
     const int ta = 2 * pr, tb = 2 * pr + 1;
     const bool hasb = tb < T;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
@@ -652,7 +656,7 @@ hipError_t launch_fwd16c(const Plan& p, const int2* cw, const unsigned short* sr
     if (p.nwave > 0) {
         const int RB = (p.nwave + WG / 64 - 1) / (WG / 64);
         const int fw = src_fires && fires_ld(src_rows) <= FIRES_LDS_WORDS ? fires_ld(src_rows) : 0;
-        const dim3 grid((unsigned)((long long)T * RB));
+        const dim3 grid((unsigned)tile_blocks(RB, T));
         const size_t lds = (size_t)(fw > 0 ? fw - 4 : 0) * 4;
         if (p.pb == 6)
             k_cfwd16<6><<<grid, WG, lds, st>>>(p, cw, src, src_rows, epi, part, T, RB, src_fires, fw);
@@ -685,7 +689,7 @@ hipError_t launch_fwd16c_lds(const Plan& p, const int2* cw, const unsigned short
             p.pb == 6 ? reinterpret_cast<const void*>(&k_cfwd16_lds<6>) : reinterpret_cast<const void*>(&k_cfwd16_lds<8>);
         const hipError_t attr = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)FWD_LDS_BYTES);
         if (attr != hipSuccess) return attr;       // (k_fwd_lds)
-        const dim3 grid((unsigned)((long long)T * S));
+        const dim3 grid((unsigned)tile_blocks(S, T));
         if (p.pb == 6)
             k_cfwd16_lds<6><<<grid, FWD_LDS_NW * 64, lds, st>>>(p, cw, (const bf16_t*)src, src_rows, epi, part, T, S);
         else
@@ -717,6 +721,7 @@ __global__ __launch_bounds__(BWD_LDS_NW * 64) void k_cbwd16_lds(Plan p, const in
     extern __shared__ __align__(16) u32x4 gs16[];          // LDS row r: slab row hot_rows[r]; row `hot`: zeros
     int s;
     const int tile = tile_of(blockIdx.x, S, T, s);
+    if (s >= S) return;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63, gi = grp & 7;
     const int w0 = __builtin_amdgcn_readfirstlane(s * BWD_LDS_NW + (int)(threadIdx.x >> 6)), dw = S * BWD_LDS_NW;
     const int n = w0 < p.nwave ? min((p.nwave - 1 - w0) / dw + 1, 64 * BWD_LDS_WREC) : 0;
@@ -961,7 +966,7 @@ hipError_t launch_bwd16c_lds(const Plan& p, const int2* wlds, const int2* cw, co
         const size_t lds = (size_t)(hot + 1) * 128;           // (and a row of zeros)
         const hipError_t attr = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (attr != hipSuccess) return attr;
-        const dim3 grid((unsigned)((long long)T * S));
+        const dim3 grid((unsigned)tile_blocks(S, T));
 #define FG_CBWD_LDS(P, K) k_cbwd16_lds<P, K><<<grid, BWD_LDS_NW * 64, lds, st>>>(p, wlds, cw, (const bf16_t*)gz, gz_rows, \
                                                                                    hot_rows, hot, gwpart, gw_ld, epi, part, T, S)
         if (p.pb == 6) {
@@ -986,10 +991,10 @@ static void launch_bwd16c_kernel(const Plan& p, const int2* cw, const unsigned s
     const int RB = (p.nwave + WG / 64 - 1) / (WG / 64);
     // a hop layer may take two tiles per workgroup; the sensory layer's epilogue leaves no VGPRs for a second
     if (MODE == 1 && pair)
-        k_cbwd16x2<1, PB><<<(unsigned)((long long)((T + 1) / 2) * RB), WG, 0, st>>>(p, cw, gz, gz_rows, gwpart, gw_ld,
+        k_cbwd16x2<1, PB><<<(unsigned)tile_blocks(RB, (T + 1) / 2), WG, 0, st>>>(p, cw, gz, gz_rows, gwpart, gw_ld,
                                                                                    epi, part, T, RB);
     else
-        k_cbwd16<MODE, PB><<<(unsigned)((long long)T * RB), WG, 0, st>>>(p, cw, gz, gz_rows, gwpart, gw_ld, epi, part, T,
+        k_cbwd16<MODE, PB><<<(unsigned)tile_blocks(RB, T), WG, 0, st>>>(p, cw, gz, gz_rows, gwpart, gw_ld, epi, part, T,
                                                                         RB);
 }
 

@@ -65,6 +65,7 @@ __global__ __launch_bounds__(WG) void k_fwd16(Plan p, const int2* __restrict__ c
     __shared__ __align__(16) int2 slots[WG / LPR][LPR];
     int rb;
     const int tile = tile_of(blockIdx.x, RB, T, rb);
+    if (rb >= RB) return;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
@@ -114,6 +115,7 @@ __global__ __launch_bounds__(WG) void k_bwd16(Plan p, const int2* __restrict__ c
     __shared__ __align__(16) int2 slots[WG / LPR][LPR];
     int rb;
     const int tile = tile_of(blockIdx.x, RB, T, rb);
+    if (rb >= RB) return;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
@@ -265,7 +267,7 @@ void fh_spmm_h(const int* wave, int nwave, const int* seg, int nseg, const int* 
     Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_rows, nslot, npos};
     if (nwave > 0) {
         const int RB = (nwave + WG / 64 - 1) / (WG / 64);
-        k_fwd16<F16><<<(unsigned)((long long)T * RB), WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)hs, n_src,
+        k_fwd16<F16><<<(unsigned)tile_blocks(RB, T), WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)hs, n_src,
                                                                   out, B, scratch, T, RB);
         FG_CHECK(hipGetLastError(), );
     }
@@ -291,7 +293,7 @@ void fh_spmm_bwd_h(const int* wave, int nwave, const int* seg, int nseg, const i
     Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_src, nslot, npos};
     if (nwave > 0) {
         const int RB = (nwave + WG / 64 - 1) / (WG / 64);
-        k_bwd16<F16><<<(unsigned)((long long)T * RB), WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)gzs, n_rows,
+        k_bwd16<F16><<<(unsigned)tile_blocks(RB, T), WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)gzs, n_rows,
                                                                   (const unsigned short*)hs, gh, B, gw ? gwpart : nullptr,
                                                                   npos, scale, scratch, T, RB);
         FG_CHECK(hipGetLastError(), );

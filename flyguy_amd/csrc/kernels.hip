@@ -132,6 +132,7 @@ __global__ __launch_bounds__(WG) void k_fwd(Plan p, const int2* __restrict__ cw,
     extern __shared__ __align__(16) unsigned fires[];     // the source rows' firing bits of this tile
     int rb;
     const int tile = tile_of(blockIdx.x, RB, T, rb);
+    if (rb >= RB) return;
     const bool bits = stage_fires(src_fires, fw_ld, tile, fires);     // (only for a tile with silent source rows)
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
@@ -198,6 +199,7 @@ __global__ __launch_bounds__(FWD_LDS_NW * 64) void k_fwd_lds(Plan p, const int2*
     extern __shared__ __align__(16) float4 xs[];          // the tile's slab, src_rows x LPR float4
     int s;
     const int tile = tile_of(blockIdx.x, S, T, s);
+    if (s >= S) return;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63, gi = grp & 7;
     const int w0 = __builtin_amdgcn_readfirstlane(s * FWD_LDS_NW + (int)(threadIdx.x >> 6)), dw = S * FWD_LDS_NW;
     const int n = w0 < p.nwave ? (p.nwave - 1 - w0) / dw + 1 : 0;
@@ -280,6 +282,7 @@ __global__ __launch_bounds__(FWD_LDS_NW * 64) void k_plug_bwd_lds(const float* _
     constexpr int G = FWD_LDS_NW * 64 / LPR;
     int s;
     const int tile = tile_of(blockIdx.x, S, T, s);
+    if (s >= S) return;
     const float4* gx = reinterpret_cast<const float4*>(x + (size_t)tile * x_rows * TW);
     for (int i = threadIdx.x; i < x_rows * LPR; i += FWD_LDS_NW * 64) xs[i] = gx[i];
     __syncthreads();
@@ -551,6 +554,7 @@ __global__ __launch_bounds__(WG) void k_bwd(Plan p, const int2* __restrict__ cw,
     __shared__ __align__(16) int2 slots[WG / LPR][LPR];
     int rb;
     const int tile = tile_of(blockIdx.x, RB, T, rb);
+    if (rb >= RB) return;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
@@ -617,6 +621,7 @@ __global__ __launch_bounds__(WG) void k_bwd2(Plan p, const int2* __restrict__ cw
     __shared__ __align__(16) int2 slots[WG / LPR][LPR];
     int rb;
     const int pr = tile_of(blockIdx.x, RB, (T + 1) / 2, rb);
+    if (rb >= RB) return;
     const int ta = 2 * pr, tb = 2 * pr + 1;
     const bool hasb = tb < T;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
@@ -754,6 +759,7 @@ __global__ __launch_bounds__(BWD_LDS_NW * 64) void k_bwd_lds(Plan p, const int2*
     extern __shared__ __align__(16) float4 gs[];          // LDS row r: slab row hot_rows[r], LPR float4
     int s;
     const int tile = tile_of(blockIdx.x, S, T, s);
+    if (s >= S) return;
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63, gi = grp & 7;
     const int w0 = __builtin_amdgcn_readfirstlane(s * BWD_LDS_NW + (int)(threadIdx.x >> 6)), dw = S * BWD_LDS_NW;
     const int n = w0 < p.nwave ? min((p.nwave - 1 - w0) / dw + 1, 64 * BWD_LDS_WREC) : 0;
@@ -1229,7 +1235,7 @@ hipError_t launch_fwd(const Plan& p, const int2* cw, const float* src, Lay ls, i
     if (p.nwave > 0) {
         const int RB = (p.nwave + WG / 64 - 1) / (WG / 64);
         const int fw = src_fires && ls.row == TW && fires_ld(src_rows) <= FIRES_LDS_WORDS ? fires_ld(src_rows) : 0;
-        const dim3 grid((unsigned)((long long)T * RB));
+        const dim3 grid((unsigned)tile_blocks(RB, T));
         const size_t lds = (size_t)(fw > 0 ? fw - 4 : 0) * 4;
         if (ls.row != TW)
             k_fwd<false, 8><<<grid, WG, 0, st>>>(p, cw, src, ls, src_rows, epi, part, lp, T, RB, nullptr, 0);
@@ -1260,7 +1266,7 @@ hipError_t launch_fwd_lds(const Plan& p, const int2* cw, const float* src, int s
         const void* k = p.pb == 6 ? reinterpret_cast<const void*>(&k_fwd_lds<6>) : reinterpret_cast<const void*>(&k_fwd_lds<8>);
         const hipError_t attr = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)FWD_LDS_BYTES);
         if (attr != hipSuccess) return attr;
-        const dim3 grid((unsigned)((long long)T * S));
+        const dim3 grid((unsigned)tile_blocks(S, T));
         if (p.pb == 6)
             k_fwd_lds<6><<<grid, FWD_LDS_NW * 64, lds, st>>>(p, cw, src, src_rows, epi, part, lp, T, S);
         else
@@ -1303,7 +1309,7 @@ hipError_t launch_plug_bwd_lds(const float* gd, const float* x, int x_rows, cons
     const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_plug_bwd_lds),    // (k_fwd_lds)
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)FWD_LDS_BYTES);
     if (attr != hipSuccess) return attr;
-    k_plug_bwd_lds<<<(unsigned)((long long)T * S), FWD_LDS_NW * 64, lds, st>>>(gd, x, x_rows, in_crow, in_col, n_s, ginb,
+    k_plug_bwd_lds<<<(unsigned)tile_blocks(S, T), FWD_LDS_NW * 64, lds, st>>>(gd, x, x_rows, in_crow, in_col, n_s, ginb,
                                                                                gb_ld, ginw, gw_ld, T, S);
     return hipGetLastError();
 }
@@ -1327,12 +1333,12 @@ static void launch_bwd_kernel(const Plan& p, const int2* cw, const float* gz, La
     const int RB = (p.nwave + WG / 64 - 1) / (WG / 64);
     if constexpr (TILED && MODE != 0) {
         if (pair) {                             // two tiles per workgroup
-            k_bwd2<MODE, PB><<<(unsigned)((long long)((T + 1) / 2) * RB), WG, 0, st>>>(p, cw, gz, lg, gz_rows, hsrc, lhs,
+            k_bwd2<MODE, PB><<<(unsigned)tile_blocks(RB, (T + 1) / 2), WG, 0, st>>>(p, cw, gz, lg, gz_rows, hsrc, lhs,
                                                                                      gwpart, gw_ld, epi, part, lp, T, RB);
             return;
         }
     }
-    k_bwd<TILED, MODE, PB><<<(unsigned)((long long)T * RB), WG, 0, st>>>(p, cw, gz, lg, gz_rows, hsrc, lhs, gwpart, gw_ld,
+    k_bwd<TILED, MODE, PB><<<(unsigned)tile_blocks(RB, T), WG, 0, st>>>(p, cw, gz, lg, gz_rows, hsrc, lhs, gwpart, gw_ld,
                                                                          epi, part, lp, T, RB);
 }
 
@@ -1424,7 +1430,7 @@ hipError_t launch_bwd_lds(const Plan& p, const int2* wlds, const int2* cw, const
         const size_t lds = (size_t)(hot + 1) * TW * 4;        // (and a row of zeros)
         const hipError_t attr = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (attr != hipSuccess) return attr;
-        const dim3 grid((unsigned)((long long)T * S));
+        const dim3 grid((unsigned)tile_blocks(S, T));
 #define FG_BWD_LDS(P, K) k_bwd_lds<P, K><<<grid, BWD_LDS_NW * 64, lds, st>>>(p, wlds, cw, gz, gz_rows, hot_rows, hot, \
                                                                                hsrc, lhs, gwpart, gw_ld, epi, part, lp, T, S)
         if (p.pb == 6) {

@@ -1,0 +1,70 @@
+"""Batches of every tile count modulo 8 (the tiles that do not come in eights are cut into slices over the XCDs):
+every row of every tile is computed exactly once."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from flyguy_amd.fly_hip import HopHip
+from flyguy_amd.synth import scaled_3hop
+from gpu_helpers import NAMES, Core, rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def net():
+    return scaled_3hop(16)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 4, 5, 6, 7, 9, 13, 16, 23, 67])
+def test_any_tile_count(gpu_lib, net, tiles, bf16):
+    """Logits bit for bit those of single tiles (a sample's sums do not depend on its batch), the gradients the sum of
+    the tiles' gradients (float32 sums in another order)."""
+    s, params = net
+    w = 64 if bf16 else 32
+    rng = np.random.default_rng(tiles)
+    obs = rng.standard_normal((tiles * w, s["obs_dim"])).astype(np.float32)
+    dl = rng.standard_normal((tiles * w, s["n_act"])).astype(np.float32)
+    core = Core(s, params, tiles * w, int(bf16))
+    core.zero_grad()
+    logits = core.forward(obs)
+    core.backward(dl)
+    got = core.get(4)
+    core.zero_grad()
+    for i in range(0, tiles * w, w):
+        assert np.array_equal(core.forward(obs[i:i + w]), logits[i:i + w]), i // w
+        core.backward(dl[i:i + w])
+    for name, a, b in zip(NAMES, got, core.get(4)):
+        # both add the same per-tile terms in float32: a few rounding errors of 6e-8 of the larger partial sums
+        assert rel(a, b) <= 2e-6, (name, rel(a, b))
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("B", [32, 96, 160, 288, 352, 416, 736])
+def test_hop_of_any_tile_count(gpu_lib, net, B, half):
+    """HopHip: product and state gradient bit for bit those of single tiles (binary16 tiles hold 64 samples; the scale of
+    the gradient is the batch's, so it is held to one shared largest value)."""
+    s, params = net
+    h = s["hop"][1]
+    put = lambda a, t: torch.as_tensor(np.ascontiguousarray(a, dtype=t)).cuda()      # noqa: E731
+    base = int(h["widx"].min())
+    index = (put(h["crow"], np.int64), put(h["col"], np.int32), put(h["tcrow"], np.int64), put(h["tcol"], np.int32),
+             put(h["twidx"] - base, np.int64))
+    weights = put(params[0][h["widx"]], np.float32)
+    g = torch.Generator(device="cuda").manual_seed(B)
+    x = torch.randn(len(h["tcrow"]) - 1, B, device="cuda", generator=g)
+    gz = torch.randn(len(h["crow"]) - 1, B, device="cuda", generator=g).clamp(-2, 2)
+    gz[0] = 2.0
+
+    def run(x, gz):
+        x, w = x.contiguous().requires_grad_(), weights.clone().requires_grad_()
+        out = HopHip.apply(w, x, *index, half)
+        return (out.detach(),) + torch.autograd.grad(out, (w, x), gz.contiguous())
+    out, gw, gh = run(x, gz)
+    parts = [run(x[:, i:i + 64], gz[:, i:i + 64]) for i in range(0, B, 64)]
+    assert torch.equal(out, torch.cat([p[0] for p in parts], 1))
+    assert torch.equal(gh, torch.cat([p[2] for p in parts], 1))
+    assert rel(gw.cpu(), sum(p[1] for p in parts).cpu()) <= 2e-6
