@@ -40,21 +40,40 @@ void clear_error();
 // Each XCD first works through whole tiles of its own, x, x+8, ..., one after another, row blocks inner, so its L2 holds
 // one tile's source slab at a time.  The T % 8 tiles left are cut into 8 slices each (slice j: row blocks j, j+8, ...,
 // an even sample of a plan sorted by length), and XCD x takes T % 8 consecutive slices, so that all XCDs get the same
-// work and each reads at most two of those slabs.  (Walking all tiles in plain order whenever T % 8 != 0 had every XCD
-// read every slab: B=416, 13 tiles, hop 1 / 2 / 3 forward 142 / 255 / 60 us, with the slices 132 / 178 / 41 us.)
+// work and each reads at most two of those slabs.  The slices of one tile are walked together, in one pass from the
+// plan's longest rows to its shortest: waves of one length walk their rows' ascending sources at one pace.  The slices
+// of two tiles are walked one tile after the other, or all in one pass (together) where the plan's lengths differ so
+// much that a second pass would begin with another chain of longest rows (Plan::stripe).
+// Walking all tiles in plain order whenever T % 8 != 0 had every XCD read every slab: B=416 (13 tiles) on the benchmark
+// network, forward 537 us, now 388; B=128 201 -> 160.  At B=416 the striped hops 1 / 2 take 135 / 174 us one tile after
+// the other and 125 / 161 together; an Erdos-Renyi network's 114 / 167 and 114 / 180, its backward 176 / 165 and 182 /
+// 177, the lognormal one's backward 173 / 166 and 178 / 175.
 // A slice may be one block short: rb >= RB is a block without work.
 __host__ __device__ inline long long tile_blocks(int RB, int T) {
     const int r = T & 7;
     return (long long)(T - r) * RB + 8LL * r * ((RB + 7) / 8);
 }
-__device__ __forceinline__ int tile_of(int bid, int RB, int T, int& rb) {
-    const int x = bid & 7, s = bid >> 3, whole = (T >> 3) * RB;
+__device__ __forceinline__ int tile_of(int bid, int RB, int T, int& rb, bool together = false) {
+    const int x = bid & 7, r = T & 7, whole = (T >> 3) * RB;
+    int s = bid >> 3;
     if (s < whole) {
         rb = s % RB;
         return x + 8 * (s / RB);
     }
-    const int per = (RB + 7) / 8, i = x * (T & 7) + (s - whole) / per;      // slice i: slice i % 8 of left tile i / 8
-    rb = (i & 7) + 8 * ((s - whole) % per);
+    s -= whole;
+    // slices i .. i + r - 1 (slice i: slice i % 8 of left tile i / 8), walked n at a time from slice i
+    int i = x * r, n = r;
+    if (!together) {
+        n = min(8 - (i & 7), r);                // the first tile's
+        const int first = n * ((RB + 7) / 8);
+        if (s >= first) {                       // the next tile's
+            s -= first;
+            i += n;
+            n = r - n;
+        }
+    }
+    i += s % n;
+    rb = (i & 7) + 8 * (s / n);
     return (T & ~7) + (i >> 3);
 }
 

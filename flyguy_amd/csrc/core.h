@@ -18,7 +18,8 @@ struct DevPlan {
     int nwave = 0, nseg = 0, nsplit = 0, nslot = 0, rows = 0;
     long long npos = 0;
     int pb = 8;                                 // pair storage (Plan::pb)
-    Plan view() const { return Plan{wave, nwave, seg, nseg, split, nsplit, rows, nslot, npos, pb}; }
+    bool stripe = false;                        // Plan::stripe
+    Plan view() const { return Plan{wave, nwave, seg, nseg, split, nsplit, rows, nslot, npos, pb, stripe}; }
 };
 
 struct HopD {

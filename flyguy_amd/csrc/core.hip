@@ -140,12 +140,26 @@ static int pair_storage(int gathered_rows, const HostPlan& h) {
     return gathered_rows <= PAIR6_MAX_ROWS && steps >= 3 * waves ? 6 : 8;
 }
 
+// Whether the forward's workgroups take one wave from each quarter of a plan instead of four in a row (Plan::stripe):
+// where the longest waves are at least four times as long as the middle one.  The long waves, which only gather, then
+// share their CUs with short ones, which mostly wait for plan records and stores, and are dealt out over four times
+// as many CUs.  Lognormal in-degrees (293 and 367 edges against about 12) at B=4096: hop 1 / 2 forward 1081 / 1398 ->
+// 1055 / 1348 us.  Where the lengths are close there is nothing to mix, and rows of one length next to each other
+// gather from nearby sources: an Erdos-Renyi hop (50 against 26) took 1008 / 1517 us in a row and 1032 / 1533 us
+// striped, hop 3 (all rows split, 72 against 55) 325 and 334 us; the backward, whose waves wait for their own rows' h
+// lines first, 1387 / 1509 in a row and 1399 / 1520 us striped, so it takes every plan in a row.
+static bool striped(const HostPlan& h) {
+    const size_t n = h.wave.size();
+    return n > 0 && h.wave[0].y >= 4 * std::max(h.wave[n / 2].y, 8);
+}
+
 // the plan on the device, with its positions resolved through col (source rows) and idx (weight index of a CSR edge;
 // nullptr: the edge itself); gathered: the rows of the state its product gathers
 static bool upload_plan(Core& c, const HostPlan& h, int rows, const std::vector<int>& col, const std::vector<int>* idx,
                         int gathered, DevPlan& d) {
     d.rows = rows;
     d.pb = pair_storage(gathered, h);
+    d.stripe = striped(h);
     d.nwave = (int)h.wave.size();
     d.nseg = (int)h.seg.size();
     d.nsplit = (int)h.split.size();

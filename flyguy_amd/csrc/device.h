@@ -42,6 +42,13 @@ __device__ __forceinline__ float dot4(const float4& a, const float4& b) {
 }
 __device__ __forceinline__ float hsum4(const float4& a) { return ((a.x + a.y) + a.z) + a.w; }
 
+// the plan wave of this wave of row block rb (of RB blocks): four in a row, or (Plan::stripe) one from each quarter of
+// the plan
+__device__ __forceinline__ int wave_of(const Plan& p, int rb, int RB) {
+    const int i = (int)(threadIdx.x >> 6);
+    return __builtin_amdgcn_readfirstlane(p.stripe ? rb + RB * i : rb * (WG / 64) + i);
+}
+
 // wave w of the plan ({woff, longest segment}); false when w is past the end or names positions outside the plan
 __device__ __forceinline__ bool load_wave(const Plan& p, int w, int2& wv) {
     wv = make_int2(0, 0);

@@ -131,11 +131,11 @@ __global__ __launch_bounds__(WG) void k_fwd(Plan p, const int2* __restrict__ cw,
     __shared__ __align__(16) int2 slots[WG / LPR][LPR];
     extern __shared__ __align__(16) unsigned fires[];     // the source rows' firing bits of this tile
     int rb;
-    const int tile = tile_of(blockIdx.x, RB, T, rb);
+    const int tile = tile_of(blockIdx.x, RB, T, rb, p.stripe);
     if (rb >= RB) return;
     const bool bits = stage_fires(src_fires, fw_ld, tile, fires);     // (only for a tile with silent source rows)
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
+    const int w = wave_of(p, rb, RB);
     int2 wv;
     const bool wok = load_wave(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
