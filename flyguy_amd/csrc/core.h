@@ -107,6 +107,7 @@ struct Core {
     // those of rows whose own output is zero on the tile.  skip_silent false (FLYGUY_SKIP_SILENT=0): neither (the
     // results are the same).
     bool skip_silent = true;
+    bool skip_always = false;        // (FLYGUY_SKIP_SILENT=1: the forward's skips at every batch, fwd_skips in core.hip)
     int plug_lds = -1;               // the plug staged in LDS: -1 by batch size, 0 never, S > 0 with S workgroups per tile
     int bwd_lds = -1;                // k_bwd_lds for the hops that have it: -1 from BWD_LDS_MIN_TILES tiles up, 0 never,
                                      //   1 at every batch (FLYGUY_BWD_LDS)

@@ -652,7 +652,10 @@ Core* build(const unsigned char* bytes, long long len, int max_batch, int prec) 
     c->info0 = dalloc<float4>(*c, c->n_s);
     c->sinfo0 = dalloc<float4>(*c, c->pp.nseg);
     if (!c->info0 || !c->sinfo0) return nullptr;
-    if (const char* f = std::getenv("FLYGUY_SKIP_SILENT")) c->skip_silent = f[0] != '0';
+    if (const char* f = std::getenv("FLYGUY_SKIP_SILENT")) {
+        c->skip_silent = f[0] != '0';
+        c->skip_always = f[0] == '1';
+    }
     if (const char* f = std::getenv("FLYGUY_PLUG_LDS")) c->plug_lds = std::min(std::max(std::atoi(f), 0), 64);
     if (!(prec ? lds_plug_fits16() : lds_plug_fits())) c->plug_lds = 0;     // (a device with less LDS per workgroup)
     for (int l = 0; l < K; ++l) {                   // (the top layer's would have no reader)
@@ -777,6 +780,17 @@ static int plug_split(const Core& c, int T, int total = 2048) {
     return T >= 64 ? std::max(1, total / T) : 0;
 }
 
+// Whether a hop's forward skips the gathers of silent source rows: the layer below then records a byte per row and a
+// launch packs them (k_fires_pack, 5 us), and on the benchmark network (8.9% silent lines) hop 2 gains 7%.  So from
+// FIRES_MIN_LINES gathered lines (about 90 us) up, and never in a launch of few tiles (fwd_deep).  Forward without /
+// with bitmaps at 6, 8, 13, 16, 32 tiles: 205 / 213, 233 / 243, 362 / 366, 417 / 422, 807 / 797 us; hop 2 alone with them
+// from 8 tiles up: 13 tiles 357, 16 tiles 414 us.  FLYGUY_SKIP_SILENT=1 takes them at every batch.
+constexpr long long FIRES_MIN_LINES = 12000000;
+static bool fwd_skips(const Core& c, const HopD& d, int T, bool bf16) {
+    if (!c.skip_silent || c.skip_always) return c.skip_silent;
+    return (long long)d.E * T >= FIRES_MIN_LINES && (bf16 || !fwd_deep(d.fp.view(), T));
+}
+
 bool forward(Core& c, const float* obs, int B, float* logits, int set) {
     if (c.prec) return forward16(c, obs, B, logits, set);
     const int T = B / TW;
@@ -789,9 +803,11 @@ bool forward(Core& c, const float* obs, int B, float* logits, int set) {
         Timed t(c, ST_PACK);
         FG_CHECK(derive_forward(c, set, false, gain, theta), false);
     }
-    // each layer below the top records which rows fire on each tile; its bitmaps are packed before the next hop
-    auto bytes = [&](int layer) { return c.skip_silent ? c.fire_bytes[(size_t)layer] : nullptr; };
-    auto bits = [&](int layer) { return c.skip_silent ? c.fire_bits[(size_t)layer] : nullptr; };
+    // a layer whose next hop skips its silent rows records which rows fire on each tile, packed into bitmaps before that
+    // hop
+    auto skips = [&](int layer) { return layer < c.hops && fwd_skips(c, c.hop[(size_t)layer], T, false); };
+    auto bytes = [&](int layer) { return skips(layer) ? c.fire_bytes[(size_t)layer] : nullptr; };
+    auto bits = [&](int layer) { return skips(layer) ? c.fire_bits[(size_t)layer] : nullptr; };
     FwdEpi e0;
     e0.bias = c.arr(set, 4);
     e0.info = c.info0;
@@ -819,7 +835,7 @@ bool forward(Core& c, const float* obs, int B, float* logits, int set) {
         else
             FG_CHECK(launch_fwd(c.pp.view(), c.in_cw, c.x, tiled(c.obs_dim), c.obs_dim, e0, c.part, tiled(c.pp.nslot), T, st),
                      false);
-        if (c.skip_silent) FG_CHECK(launch_fires_pack(bytes(0), c.n_s, bits(0), T, st), false);
+        if (skips(0)) FG_CHECK(launch_fires_pack(bytes(0), c.n_s, bits(0), T, st), false);
     }
     const float* hp = c.h0;
     int hk = 0;
@@ -830,12 +846,11 @@ bool forward(Core& c, const float* obs, int B, float* logits, int set) {
         if (d.has_drive) { e.drive = c.drive; e.ldrive = tiled(c.n_s); }
         e.h = d.h; e.lh = tiled(d.rows);
         if (c.keep_z) { e.z = d.zk; e.lz = tiled(d.rows); }
-        const bool record = hk + 1 < c.hops;
-        if (record) e.fires = bytes(hk + 1);
+        e.fires = bytes(hk + 1);
         {
             Timed t(c, ST_HOP + std::min(hk, 7));
             FG_CHECK(launch_fwd(d.fp.view(), d.cw, hp, tiled(d.src), d.src, e, c.part, tiled(d.fp.nslot), T, st, bits(hk)), false);
-            if (record && c.skip_silent) FG_CHECK(launch_fires_pack(bytes(hk + 1), d.rows, bits(hk + 1), T, st), false);
+            if (skips(hk + 1)) FG_CHECK(launch_fires_pack(bytes(hk + 1), d.rows, bits(hk + 1), T, st), false);
         }
         hp = d.h;
         ++hk;
@@ -967,8 +982,9 @@ static bool forward16(Core& c, const float* obs, int B, float* logits, int set) 
         Timed t(c, ST_PACK);
         FG_CHECK(derive_forward(c, set, true, gain, theta), false);
     }
-    auto bytes = [&](int layer) { return c.skip_silent ? c.fire_bytes[(size_t)layer] : nullptr; };   // (as forward)
-    auto bits = [&](int layer) { return c.skip_silent ? c.fire_bits[(size_t)layer] : nullptr; };
+    auto skips = [&](int layer) { return layer < c.hops && fwd_skips(c, c.hop[(size_t)layer], T, true); };   // (as forward)
+    auto bytes = [&](int layer) { return skips(layer) ? c.fire_bytes[(size_t)layer] : nullptr; };
+    auto bits = [&](int layer) { return skips(layer) ? c.fire_bits[(size_t)layer] : nullptr; };
     FwdEpi16 e0;
     e0.bias = c.arr(set, 4);
     e0.info = c.info0;
@@ -983,7 +999,7 @@ static bool forward16(Core& c, const float* obs, int B, float* logits, int set) 
             FG_CHECK(launch_fwd16c_lds(c.pp.view(), c.in_cw, s16(c.x), c.obs_dim, e0, c.part, T, S, st), false);
         else
             FG_CHECK(launch_fwd16c(c.pp.view(), c.in_cw, s16(c.x), c.obs_dim, e0, c.part, T, st), false);
-        if (c.skip_silent) FG_CHECK(launch_fires_pack(bytes(0), c.n_s, bits(0), T, st), false);
+        if (skips(0)) FG_CHECK(launch_fires_pack(bytes(0), c.n_s, bits(0), T, st), false);
     }
     const u16* hp = s16(c.h0);
     int hk = 0;
@@ -995,12 +1011,11 @@ static bool forward16(Core& c, const float* obs, int B, float* logits, int set) 
         e.h = s16(d.h);
         if (c.keep_z) e.z = s16(d.zk);
         e.rows = d.rows;
-        const bool record = hk + 1 < c.hops;
-        if (record) e.fires = bytes(hk + 1);
+        e.fires = bytes(hk + 1);
         {
             Timed t(c, ST_HOP + std::min(hk, 7));
             FG_CHECK(launch_fwd16c(d.fp.view(), d.cw, hp, d.src, e, c.part, T, st, bits(hk)), false);
-            if (record && c.skip_silent) FG_CHECK(launch_fires_pack(bytes(hk + 1), d.rows, bits(hk + 1), T, st), false);
+            if (skips(hk + 1)) FG_CHECK(launch_fires_pack(bytes(hk + 1), d.rows, bits(hk + 1), T, st), false);
         }
         hp = s16(d.h);
         ++hk;

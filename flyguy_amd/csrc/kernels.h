@@ -126,8 +126,15 @@ constexpr int PACK_JOBS = 4;
 hipError_t launch_pack_n(const PackJob* jobs, int n, hipStream_t st, bool bf16w = false);
 // src_rows / gz_rows: rows of the gathered state (a gather of a row outside it reads zeros).  src_fires: the source
 // layer's firing bitmaps (launch_fires_pack; fires_ld(src_rows) words per tile; tiled states only), or nullptr
+// (a tiled launch that fwd_deep names, without bitmaps, takes k_fwd_deep)
 hipError_t launch_fwd(const Plan& p, const int2* cw, const float* src, Lay ls, int src_rows, const FwdEpi& epi,
                       float* part, Lay lp, int T, hipStream_t st, const unsigned* src_fires = nullptr);
+// Whether a tiled forward launch goes through k_fwd_deep: up to 16 plan waves a SIMD in all (256 CUs of 4 SIMDs).  Benchmark
+// network, k_fwd / k_fwd_deep: hop 1 at 1, 2, 3, 4, 5 tiles (5,800 plan waves each) 37 / 28, 41 / 34, 46 / 44, 50 / 53,
+// 59 / 63 us; hop 2 (4,750) 50 / 33, 54 / 40, 61 / 53, 63 / 62, 76 / 84; hop 3 (560) at 8, 13, 16 tiles 34 / 33, 51 /
+// 47, 54 / 53 us.  Striped plans of up to 6 waves a SIMD have four steps in flight instead of two.
+constexpr long long FWD_DEEP_WAVES = 16 * 1024, FWD_DEEP4_WAVES = 6 * 1024;
+inline bool fwd_deep(const Plan& p, int T) { return (long long)p.nwave * T <= FWD_DEEP_WAVES; }
 // Tables to bring into every XCD's L2 ahead of a kernel (launch_touch): n[k] 16-byte words at p[k] (n 0: none)
 constexpr int TOUCH_JOBS = 4;
 struct TouchJob {

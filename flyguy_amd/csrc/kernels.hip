@@ -10,6 +10,7 @@
 // reach the 8 lanes of each group through LDS; the 8 source rows are then gathered as independent 128-byte lines
 // of the tile's slab, with no branch per edge (unused positions gather NO_ROW, which reads zeros).
 #include <initializer_list>
+#include <type_traits>
 
 #include "device.h"
 #include "readout.h"
@@ -175,6 +176,89 @@ __global__ __launch_bounds__(WG) void k_fwd(Plan p, const int2* __restrict__ cw,
         in = fwd_inputs(epi, epi.sinfo ? epi.sinfo + 8 * w : nullptr, grp & 7, sg.z, tile, sub);
         if (epi.bias) acc = splat(epi.sinfo ? in.b : epi.bias[sg.x]);
     }
+    if (!live) return;
+    if (sg.y >= 0) {
+        *at4w(part, lp, tile, sg.y, sub) = acc;
+        return;
+    }
+    fwd_finish(epi, sg.x, tile, sub, acc, in);
+}
+
+// k_fwd for a batch of few tiles (fwd_deep).  There the launch is over when its longest waves are: at one tile all waves
+// fit the chip at once, and a wave of the cap's 367 edges is a chain of 46 steps, each waiting for its gathers.  This
+// kernel issues the gathers of U steps before the first is used, and takes one wave per workgroup so that the long
+// waves, which come first in the plan, are dealt out over all CUs instead of four to a CU.  The sums are k_fwd's, term
+// for term.  It reads no firing bitmaps.
+// One tile of the benchmark network, hop 1 / 2 / 3 with their combines: k_fwd 37 / 50 / 23 us with bitmaps (10 us of it
+// the packing); U = 1 32 / 38 / 19, U = 2 28 / 33 / 18, U = 4 26 / 30 / 18, U = 8 33 / 34 / 18 us (256 VGPRs, one wave a
+// SIMD); the plug (2 steps a wave) 10.6 us by k_fwd, 9.8 at U = 1 and 2, 11.1 at U = 4.
+template <int PB, int U>
+__global__ __launch_bounds__(64) void k_fwd_deep(Plan p, const int2* __restrict__ cw, const float* __restrict__ src,
+                                                 int src_rows, FwdEpi epi, float* __restrict__ part, Lay lp, int T) {
+    __shared__ __align__(16) int2 slots[U][RPW][LPR];
+    int w;
+    const int tile = tile_of(blockIdx.x, p.nwave, T, w, p.stripe);
+    if (w >= p.nwave) return;
+    const int lane = threadIdx.x, grp = lane >> 3, sub = lane & 7;
+    int2 wv;
+    const bool wok = load_wave(p, w, wv);
+    const int steps = wok ? (wv.y + 7) / 8 : 0;
+    const PairLoad<PB> q(cw, wv.x, lane);
+    int2 nxt[U];
+    if (steps > 0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) nxt[u] = q.step(min(u, steps - 1));
+    }
+    int4 sg;
+    const bool live = load_segment(p, w * 8 + grp, sg) && wok;
+    const bool whole = live && sg.y < 0;
+    const Slab<true> slab(src + (size_t)tile * src_rows * TW, TW, src_rows, sub);
+    float4 acc = splat(0.f);
+    FwdIn in{};
+    auto inputs = [&]() {                       // the row's own inputs; the bias starts the sum
+        if (!whole) return;
+        in = fwd_inputs(epi, epi.sinfo ? epi.sinfo + 8 * w : nullptr, grp, sg.z, tile, sub);
+        if (epi.bias) acc = splat(epi.sinfo ? in.b : epi.bias[sg.x]);
+    };
+    // steps j .. j + N - 1 (those past the wave's last gather nothing), their pairs in nxt
+    auto round = [&](auto n, int j) __attribute__((always_inline)) {
+        constexpr int N = decltype(n)::value;
+        float4 v[N][8];
+        float wt[N][8];
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            int c[8];
+            stage_pairs<PB>(slots[u], grp, sub, nxt[u], false, nullptr, src_rows, c, wt[u]);
+            const bool real = j + u < steps;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) v[u][s] = slab.get(real ? c[s] : NO_ROW, sub);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) nxt[u] = q.step(min(j + N + u, steps - 1));
+        if (j == 0) inputs();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+            if (j + u < steps) {
+#pragma unroll
+                for (int s = 0; s < 8; ++s) fma4(wt[u][s], v[u][s], acc);
+            }
+    };
+    int j = 0;
+    for (; j + U <= steps; j += U) round(std::integral_constant<int, U>{}, j);
+    if (j < steps) {                            // the last steps: the next power of two of them
+        const int r = steps - j;
+        if (r == 1)
+            round(std::integral_constant<int, 1>{}, j);
+        else if (r == 2)
+            round(std::integral_constant<int, 2>{}, j);
+        else if (U > 4 && r <= 4)
+            round(std::integral_constant<int, 4>{}, j);
+        else
+            round(std::integral_constant<int, U>{}, j);
+    }
+    if (steps == 0) inputs();
     if (!live) return;
     if (sg.y >= 0) {
         *at4w(part, lp, tile, sg.y, sub) = acc;
@@ -1232,7 +1316,19 @@ hipError_t launch_fwd(const Plan& p, const int2* cw, const float* src, Lay ls, i
     // 6-byte pairs name rows by 16 bits: only a tiled slab of at most PAIR6_MAX_ROWS rows reads 0xFFFF as past its end
     if ((p.pb != 8 && p.pb != 6) || (p.pb == 6 && (ls.row != TW || src_rows > PAIR6_MAX_ROWS)))
         return hipErrorInvalidValue;
-    if (p.nwave > 0) {
+    if (p.nwave > 0 && ls.row == TW && !src_fires && fwd_deep(p, T)) {
+        const unsigned grid = (unsigned)tile_blocks(p.nwave, T);
+        const int U = p.stripe && (long long)p.nwave * T <= FWD_DEEP4_WAVES ? 4 : 2;
+#define FG_FWD_DEEP(P, N) k_fwd_deep<P, N><<<grid, 64, 0, st>>>(p, cw, src, src_rows, epi, part, lp, T)
+        if (p.pb == 6) {
+            if (U == 4) FG_FWD_DEEP(6, 4); else FG_FWD_DEEP(6, 2);
+        } else {
+            if (U == 4) FG_FWD_DEEP(8, 4); else FG_FWD_DEEP(8, 2);
+        }
+#undef FG_FWD_DEEP
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    } else if (p.nwave > 0) {
         const int RB = (p.nwave + WG / 64 - 1) / (WG / 64);
         const int fw = src_fires && ls.row == TW && fires_ld(src_rows) <= FIRES_LDS_WORDS ? fires_ld(src_rows) : 0;
         const dim3 grid((unsigned)tile_blocks(RB, T));

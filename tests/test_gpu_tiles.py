@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from flyguy_amd.fly_hip import HopHip
-from flyguy_amd.synth import scaled_3hop
+from flyguy_amd.synth import scaled_3hop, synth_3hop
 from gpu_helpers import NAMES, Core, rel
 
 pytestmark = pytest.mark.gpu
@@ -68,3 +68,27 @@ def test_hop_of_any_tile_count(gpu_lib, net, B, half):
     assert torch.equal(out, torch.cat([p[0] for p in parts], 1))
     assert torch.equal(gh, torch.cat([p[2] for p in parts], 1))
     assert rel(gw.cpu(), sum(p[1] for p in parts).cpu()) <= 2e-6
+
+
+@pytest.fixture(scope="module")
+def uneven():
+    """A network whose first hop's plan has waves of 1 to 10 steps, the longest four times the middle one."""
+    return synth_3hop(sizes=(3000, 20000, 500, 40), edges=(300_000, 9_000, 900), redrive=(300, 20, 2), sigma=2.5)
+
+
+@pytest.mark.parametrize("tiles", [1, 2, 3, 5, 7, 12])
+def test_few_tiles(gpu_lib, uneven, monkeypatch, tiles):
+    """Batches of few tiles (several steps' gathers in flight, one wave per workgroup, four steps on the uneven hop up
+    to 2 tiles) against the kernel of larger batches, which firing bitmaps at every batch select: logits and every
+    layer's states bit for bit."""
+    s, params = uneven
+    B = 32 * tiles
+    obs = np.random.default_rng(tiles).standard_normal((B, s["obs_dim"])).astype(np.float32)
+    got = []
+    for mode in ("", "1"):
+        if mode:
+            monkeypatch.setenv("FLYGUY_SKIP_SILENT", mode)
+        core = Core(s, params, B)
+        got.append([core.forward(obs)] + [core.state(k, 0, n, B) for k, n in enumerate(s["sizes"])])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
