@@ -122,7 +122,14 @@ struct Core {
         bool same(int s, unsigned long long v) const { return set == s && ver == v; }
     };
     unsigned long long wver[2] = {1, 1};
-    Stamp made_fpairs, made_info, made_owT, made_tpairs;
+    // The tables in the order of their jobs (DeriveJob), each group a run of blocks: group g's are [dblock[g], dblock[g + 1])
+    enum Table { T_FPAIRS = 0, T_INFO = 1, T_OWT = 2, T_TPAIRS = 3, T_COUNT = 4 };
+    Stamp made[T_COUNT];
+    bool tables_old = false;         // a forward has run since the forward's tables were made (launch_touch)
+    DeriveJob* djobs = nullptr;
+    int* dfirst = nullptr;           // per job its first block
+    int dn_jobs = 0;
+    long long dblock[T_COUNT + 1] = {0};
     void weights_written(int set) { if (set == 0 || set == 1) ++wver[set]; }
     std::vector<unsigned char*> fire_bytes;
     std::vector<unsigned*> fire_bits;
@@ -177,6 +184,10 @@ bool forward(Core& c, const float* obs, int B, float* logits, int set);
 // fresh: the gradient arrays are zero and this backward is the only one adding to them (a teaching step), so the
 // first sum into each entry is stored instead of added (no read of the entry)
 bool backward(Core& c, const float* dlogits, int B, bool fresh = false);
+// Makes the tables that passes derive from the weights and that are not current: the forward's (from `set`) and / or
+// the backward's (from the weights, so with bwd the set is SET_P).  forward() and backward() call it for their own; a
+// step that runs both calls it for both first, in one launch.
+bool derive(Core& c, int set, bool fwd, bool bwd);
 float grad_norm(Core& c);
 // Adam + running average over all seven arrays; lr for W, lr_neuron for gain / theta, lr_plug for the rest
 float step(Core& c, float lr, float lr_neuron, float lr_plug, float max_norm, float ema);

@@ -493,6 +493,8 @@ static bool plan_net(const NetHost& n, NetPlans& p) {
     return true;
 }
 
+static bool plan_tables(Core& c);
+
 Core* build(const unsigned char* bytes, long long len, int max_batch, int prec) {
     clear_error();
     if (!bytes || len < 36 || std::memcmp(bytes, "FLY1", 4) != 0) {
@@ -683,6 +685,7 @@ Core* build(const unsigned char* bytes, long long len, int max_batch, int prec) 
         !c->gwpart || !c->ggp0 || !c->gsp0 || !c->ginb || !c->ginw || !c->gow_p || !c->gob_p || !c->stats_part ||
         !c->stats || !c->red || !c->nrm || !c->owT || !c->lpart)
         return nullptr;
+    if (!plan_tables(*c)) return nullptr;
     if (hipDeviceSynchronize() != hipSuccess) { set_error("device error after set-up"); return nullptr; }
     return c.release();
 }
@@ -699,69 +702,94 @@ bool check_batch(const Core* c, int B) {
 }
 
 // ------------------------------------------------------------------------------------------------ passes
-// the per-row neuron records of every layer from this set's gain and theta
-static hipError_t rowinfo(Core& c, const float* gain, const float* theta, const float* bias) {
-    std::vector<RowJob> j;
-    j.push_back({c.n0, nullptr, c.info0, c.n_s, nullptr, bias});          // (the plug's rows carry their bias)
-    j.push_back({c.n0, nullptr, c.sinfo0, c.pp.nseg, c.pp.seg, bias});
+bool derive(Core& c, int set, bool fwd, bool bwd) {
+    Timed t(c, ST_PACK);
+    const bool want[Core::T_COUNT] = {fwd, true, true, bwd};
+    const Core::Stamp now{set, c.wver[set]};
+    bool stale[Core::T_COUNT];
+    for (int g = 0; g < Core::T_COUNT; ++g) stale[g] = want[g] && !c.made[g].same(now.set, now.ver);
+    for (int g = 0; g < Core::T_COUNT; ++g) {
+        if (!stale[g]) continue;
+        int e = g + 1;
+        while (e < Core::T_COUNT && stale[e]) ++e;          // (neighbouring groups in one launch)
+        FG_CHECK(launch_derive(c.djobs, c.dfirst, c.dn_jobs, c.dblock[g], c.dblock[e] - c.dblock[g], c.arr(set, 0),
+                               c.arr(set, 1), c.arr(set, 2), c.prec != 0, c.st), false);
+        for (int k = g; k < e; ++k) c.made[k] = now;
+        if (g == Core::T_FPAIRS) c.tables_old = false;
+        g = e - 1;
+    }
+    return true;
+}
+
+// the jobs of every derived table, and the parts of the packed pairs that no weight changes (the 6-byte pairs' sources)
+static bool plan_tables(Core& c) {
+    std::vector<DeriveJob> j;
+    std::vector<int> first;
+    long long nb = 0;
+    auto add = [&](const DeriveJob& job) {
+        j.push_back(job);
+        first.push_back((int)nb);
+        nb += derive_blocks(job);
+    };
+    auto pairs = [&](const DevPlan& p, const int* col, int2* out, long long w) {
+        DeriveJob d;
+        d.kind = p.pb == 6 ? DeriveJob::WEIGHTS6 : DeriveJob::PAIRS8;
+        d.n = p.npos;
+        d.idx = p.pidx;
+        d.col = col;
+        d.out = out;
+        d.w = w;
+        add(d);
+        return p.pb != 6 || launch_pack(col, p.pidx, c.arr(SET_P, 0) + w, out, p.npos, nullptr, 6) == hipSuccess;
+    };
+    auto records = [&](const int* nid, const int* drow, const int4* seg, int n, float4* out, long long bias) {
+        DeriveJob d;
+        d.kind = DeriveJob::RECORDS;
+        d.n = n;
+        d.idx = nid;
+        d.col = drow;
+        d.seg = seg;
+        d.out = out;
+        d.w = bias;
+        add(d);
+    };
+    bool ok = pairs(c.pp, c.pp.pcol, c.in_cw, c.off[3]);
+    for (auto& d : c.hop) ok = ok && pairs(d.fp, d.fp.pcol, d.cw, c.off[0]);
+    c.dblock[Core::T_INFO] = nb;
+    records(c.n0, nullptr, nullptr, c.n_s, c.info0, c.off[4]);            // (the plug's rows carry their bias)
+    records(c.n0, nullptr, c.pp.seg, c.pp.nseg, c.sinfo0, c.off[4]);
     for (size_t k = 0; k < c.hop.size(); ++k) {
         HopD& d = c.hop[k];
-        j.push_back({d.nid, d.has_drive ? d.drow : nullptr, d.info, d.rows});
-        j.push_back({d.nid, d.has_drive ? d.drow : nullptr, d.sinfo, d.fp.nseg, d.fp.seg});
+        const int* drow = d.has_drive ? d.drow : nullptr;
+        records(d.nid, drow, nullptr, d.rows, d.info, -1);
+        records(d.nid, drow, d.fp.seg, d.fp.nseg, d.sinfo, -1);
         // the backward of hop k + 1 finishes the rows of the layer below (its transposed plan's rows)
-        j.push_back({k ? c.hop[k - 1].nid : c.n0, nullptr, d.bsinfo, d.bp.nseg, d.bp.seg});
+        records(k ? c.hop[k - 1].nid : c.n0, nullptr, d.bp.seg, d.bp.nseg, d.bsinfo, -1);
     }
-    hipError_t e = hipSuccess;
-    for (size_t k = 0; k < j.size() && e == hipSuccess; k += ROW_JOBS)
-        e = launch_rowinfo_n(j.data() + k, (int)std::min<size_t>(ROW_JOBS, j.size() - k), gain, theta, c.st);
-    return e;
-}
-
-// the packed (source, weight) pairs of the forward plans (plug and hops) or of the hops' transposed plans, in launches
-// of up to PACK_JOBS plans
-static hipError_t pack(Core& c, int set, bool transposed, bool bf16w) {
-    std::vector<PackJob> j;
-    const float* W = c.arr(set, 0);
-    if (!transposed) j.push_back({c.pp.pcol, c.pp.pidx, c.arr(set, 3), c.in_cw, c.pp.npos, c.pp.pb});
+    c.dblock[Core::T_OWT] = nb;
+    DeriveJob o;
+    o.kind = DeriveJob::TRANSPOSE;
+    o.rows = c.n_act;
+    o.cols = c.n_dn;
+    o.ma = readout_pad(c.n_act);
+    o.n = (long long)c.n_dn * o.ma;
+    o.out = c.owT;
+    o.w = c.off[5];
+    add(o);
+    c.dblock[Core::T_TPAIRS] = nb;
     for (auto& d : c.hop) {
-        j.push_back(transposed ? PackJob{d.bp.pcol, d.bp.pidx, W, d.tcw, d.bp.npos, d.bp.pb}
-                               : PackJob{d.fp.pcol, d.fp.pidx, W, d.cw, d.fp.npos, d.fp.pb});
-        if (transposed && d.lds_hot)    // (the same pairs with LDS codes, for k_bwd_lds)
-            j.push_back(PackJob{d.pcol_lds, d.bp.pidx, W, d.tcw_lds, d.bp.npos, d.bp.pb});
+        ok = ok && pairs(d.bp, d.bp.pcol, d.tcw, c.off[0]);
+        if (d.lds_hot) ok = ok && pairs(d.bp, d.pcol_lds, d.tcw_lds, c.off[0]);   // (with LDS codes, for k_bwd_lds)
     }
-    hipError_t e = hipSuccess;
-    for (size_t k = 0; k < j.size() && e == hipSuccess; k += PACK_JOBS)
-        e = launch_pack_n(j.data() + k, (int)std::min<size_t>(PACK_JOBS, j.size() - k), c.st, bf16w);
-    return e;
-}
-
-// The forward's packed pairs and per-row records from `set`, unless they were made from its current version
-static hipError_t derive_forward(Core& c, int set, bool bf16w, const float* gain, const float* theta) {
-    if (!c.made_fpairs.same(set, c.wver[set])) {
-        const hipError_t e = pack(c, set, false, bf16w);
-        if (e != hipSuccess) return e;
-        c.made_fpairs = {set, c.wver[set]};
+    c.dblock[Core::T_COUNT] = nb;
+    if (!ok || nb > 0x7FFFFFFFLL) {
+        set_error("derived tables");
+        return false;
     }
-    if (!c.made_info.same(set, c.wver[set])) {
-        const hipError_t e = rowinfo(c, gain, theta, c.arr(set, 4));
-        if (e != hipSuccess) return e;
-        c.made_info = {set, c.wver[set]};
-    }
-    return hipSuccess;
-}
-// The backward's transposed pairs and per-row records from the weights (SET_P), unless current
-static hipError_t derive_backward(Core& c, bool bf16w, const float* gain, const float* theta) {
-    if (!c.made_tpairs.same(SET_P, c.wver[SET_P])) {
-        const hipError_t e = pack(c, SET_P, true, bf16w);
-        if (e != hipSuccess) return e;
-        c.made_tpairs = {SET_P, c.wver[SET_P]};
-    }
-    if (!c.made_info.same(SET_P, c.wver[SET_P])) {
-        const hipError_t e = rowinfo(c, gain, theta, c.arr(SET_P, 4));
-        if (e != hipSuccess) return e;
-        c.made_info = {SET_P, c.wver[SET_P]};
-    }
-    return hipSuccess;
+    c.dn_jobs = (int)j.size();
+    c.djobs = upload(c, j);
+    c.dfirst = upload(c, first);
+    return c.djobs && c.dfirst;
 }
 
 static bool forward16(Core& c, const float* obs, int B, float* logits, int set);
@@ -796,13 +824,9 @@ bool forward(Core& c, const float* obs, int B, float* logits, int set) {
     const int T = B / TW;
     hipStream_t st = c.st;
     { Timed t(c, ST_OBS); FG_CHECK(launch_obs_in(obs, c.x, c.obs_dim, B, st), false); }
-    const float *gain = c.arr(set, 1), *theta = c.arr(set, 2);
-    // tables made in an earlier pass: the caches have moved on since (see the plug below)
-    const bool old_tables = c.made_fpairs.same(set, c.wver[set]) && c.made_info.same(set, c.wver[set]);
-    {
-        Timed t(c, ST_PACK);
-        FG_CHECK(derive_forward(c, set, false, gain, theta), false);
-    }
+    if (!derive(c, set, true, false)) return false;
+    const bool old_tables = c.tables_old;       // (the caches have moved on since they were made: see the plug below)
+    c.tables_old = true;
     // a layer whose next hop skips its silent rows records which rows fire on each tile, packed into bitmaps before that
     // hop
     auto skips = [&](int layer) { return layer < c.hops && fwd_skips(c, c.hop[(size_t)layer], T, false); };
@@ -857,9 +881,8 @@ bool forward(Core& c, const float* obs, int B, float* logits, int set) {
     }
     {
         Timed t(c, ST_LOGITS);
-        FG_CHECK(launch_logits_mfma(hp, false, c.sizes[c.hops], c.dn, c.n_dn, c.arr(set, 5), c.arr(set, 6), c.n_act, c.owT,
-                                    c.lpart, logits, B, st, c.made_owT.same(set, c.wver[set])), false);
-        c.made_owT = {set, c.wver[set]};
+        FG_CHECK(launch_logits_mfma(hp, false, c.sizes[c.hops], c.dn, c.n_dn, c.arr(set, 6), c.n_act, c.owT, c.lpart, logits,
+                                    B, st), false);
     }
     c.B = B;
     return true;
@@ -869,13 +892,10 @@ bool backward(Core& c, const float* dlogits, int B, bool fresh) {
     if (c.prec) return backward16(c, dlogits, B, fresh);
     const int T = B / TW, K = c.hops;
     hipStream_t st = c.st;
-    const float *gain = c.arr(SET_P, 1), *theta = c.arr(SET_P, 2);
+    const float* theta = c.arr(SET_P, 2);
     float* G[7];
     for (int i = 0; i < 7; ++i) G[i] = c.arr(SET_G, i);
-    {
-        Timed t(c, ST_PACK);
-        FG_CHECK(derive_backward(c, false, gain, theta), false);
-    }
+    if (!derive(c, SET_P, false, true)) return false;
 
     HopD& top = c.hop[K - 1];
     BwdEpi et;
@@ -889,10 +909,6 @@ bool backward(Core& c, const float* dlogits, int B, bool fresh) {
     et.ggain_part = top.ggp; et.gsum_part = top.gsp; et.gp_ld = top.rows;
     {
         Timed t(c, ST_RBWD);
-        if (!c.made_owT.same(SET_P, c.wver[SET_P])) {
-            FG_CHECK(launch_owT(c.arr(SET_P, 5), c.n_act, c.n_dn, c.owT, st), false);
-            c.made_owT = {SET_P, c.wver[SET_P]};
-        }
         FG_CHECK(launch_readout_bwd_h_mfma(dlogits, c.owT, c.dn_inv, c.n_act, top.rows, et, B, st), false);
         FG_CHECK(launch_readout_bwd_w_mfma(dlogits, top.h, false, top.rows, c.dn, c.n_dn, c.n_act, c.gow_p, c.gob_p, B, st),
                  false);
@@ -977,11 +993,7 @@ static bool forward16(Core& c, const float* obs, int B, float* logits, int set) 
     const int T = B / TW16;
     hipStream_t st = c.st;
     { Timed t(c, ST_OBS); FG_CHECK(launch_obs_in16(obs, s16(c.x), c.obs_dim, B, st), false); }
-    const float *gain = c.arr(set, 1), *theta = c.arr(set, 2);
-    {
-        Timed t(c, ST_PACK);
-        FG_CHECK(derive_forward(c, set, true, gain, theta), false);
-    }
+    if (!derive(c, set, true, false)) return false;
     auto skips = [&](int layer) { return layer < c.hops && fwd_skips(c, c.hop[(size_t)layer], T, true); };   // (as forward)
     auto bytes = [&](int layer) { return skips(layer) ? c.fire_bytes[(size_t)layer] : nullptr; };
     auto bits = [&](int layer) { return skips(layer) ? c.fire_bits[(size_t)layer] : nullptr; };
@@ -1022,9 +1034,8 @@ static bool forward16(Core& c, const float* obs, int B, float* logits, int set) 
     }
     {
         Timed t(c, ST_LOGITS);
-        FG_CHECK(launch_logits_mfma(hp, true, c.sizes[c.hops], c.dn, c.n_dn, c.arr(set, 5), c.arr(set, 6), c.n_act, c.owT,
-                                    c.lpart, logits, B, st, c.made_owT.same(set, c.wver[set])), false);
-        c.made_owT = {set, c.wver[set]};
+        FG_CHECK(launch_logits_mfma(hp, true, c.sizes[c.hops], c.dn, c.n_dn, c.arr(set, 6), c.n_act, c.owT, c.lpart, logits,
+                                    B, st), false);
     }
     c.B = B;
     return true;
@@ -1033,13 +1044,10 @@ static bool forward16(Core& c, const float* obs, int B, float* logits, int set) 
 static bool backward16(Core& c, const float* dlogits, int B, bool fresh) {
     const int T = B / TW16, K = c.hops;
     hipStream_t st = c.st;
-    const float *gain = c.arr(SET_P, 1), *theta = c.arr(SET_P, 2);
+    const float* theta = c.arr(SET_P, 2);
     float* G[7];
     for (int i = 0; i < 7; ++i) G[i] = c.arr(SET_G, i);
-    {
-        Timed t(c, ST_PACK);
-        FG_CHECK(derive_backward(c, true, gain, theta), false);
-    }
+    if (!derive(c, SET_P, false, true)) return false;
     HopD& top = c.hop[K - 1];
     BwdEpi16 et;
     et.mode = 1;
@@ -1054,10 +1062,6 @@ static bool backward16(Core& c, const float* dlogits, int B, bool fresh) {
     et.ggain_part = top.ggp; et.gsum_part = top.gsp; et.gp_ld = top.rows;
     {
         Timed t(c, ST_RBWD);
-        if (!c.made_owT.same(SET_P, c.wver[SET_P])) {
-            FG_CHECK(launch_owT(c.arr(SET_P, 5), c.n_act, c.n_dn, c.owT, st), false);
-            c.made_owT = {SET_P, c.wver[SET_P]};
-        }
         FG_CHECK(launch_readout_bwd_h16_mfma(dlogits, c.owT, c.dn_inv, c.n_act, top.rows, et, B, st), false);
         FG_CHECK(launch_readout_bwd_w_mfma(dlogits, top.h, true, top.rows, c.dn, c.n_dn, c.n_act, c.gow_p, c.gob_p, B, st),
                  false);
@@ -1198,7 +1202,7 @@ void fc_set_stream(void* h, void* stream) {
     Core* c = (Core*)h;
     if (!c) return;
     if (c->st != (hipStream_t)stream)           // (tables made on another stream are made again on this one)
-        c->made_fpairs = c->made_info = c->made_owT = c->made_tpairs = Core::Stamp{};
+        for (auto& m : c->made) m = Core::Stamp{};
     c->st = (hipStream_t)stream;
 }
 
@@ -1276,7 +1280,7 @@ float fc_teach_step(void* h, const float* obs, const float* teacher, int B, floa
     if (!check_batch(c, B)) return -1.f;
     if (!obs || !teacher) { set_error("fc_teach_step: null pointer"); return -1.f; }
     { Timed t(*c, ST_ZERO); FG_CHECK(launch_fill(c->arr(SET_G, 0), 0.f, c->PT, c->st), -1.f); }
-    if (!forward(*c, obs, B, c->lg, SET_P)) return -1.f;
+    if (!derive(*c, SET_P, true, true) || !forward(*c, obs, B, c->lg, SET_P)) return -1.f;
     {
         Timed t(*c, ST_LOSS);
         FG_CHECK(launch_loss(c->lg, teacher, c->dl, c->stats_part, stats ? stats : c->stats, c->n_act, B, it, c->st), -1.f);

@@ -110,20 +110,32 @@ struct BwdEpi {
 };
 
 // launch wrappers (all asynchronous on `st`)
-// cw[p] = (pcol[p], w[pidx[p]]) for the npos positions of a plan; pidx[p] < 0: (NO_ROW, 0).  bf16w: the weight
-// rounded to bfloat16 (nearest even), as the float32 of that value (the bfloat16-state core's products)
+// cw[p] = (pcol[p], w[pidx[p]]) for the npos positions of a plan; pidx[p] < 0: (NO_ROW, 0)
 hipError_t launch_pack(const int* pcol, const int* pidx, const float* w, int2* cw, long long npos, hipStream_t st,
-                       bool bf16w = false);
-// the same for up to PACK_JOBS plans in one launch
-struct PackJob {
-    const int *pcol = nullptr, *pidx = nullptr;
-    const float* w = nullptr;
-    int2* cw = nullptr;
-    long long n = 0;
-    int pb = 8;                       // the plan's pair storage (Plan::pb); 6 takes n a multiple of 64
+                       int pb = 8);   // pb 6 (Plan::pb): npos a multiple of 64
+// The tables a pass derives from one set of weights, a job each (k_derive).  A job's weights are given by their offset
+// in the set (floats); npos of a pair job is a multiple of 64.
+struct DeriveJob {
+    enum Kind { PAIRS8 = 0, WEIGHTS6 = 1, RECORDS = 2, TRANSPOSE = 3 };
+    int kind = PAIRS8;
+    // PAIRS8: out[p] = (col[p], w[idx[p]]), idx < 0: (NO_ROW, 0).  WEIGHTS6: the weight planes of 6-byte pairs (their
+    // source planes never change: launch_pack writes them once).  RECORDS: per row r (or per segment, row = seg.x) of a
+    // layer {gain[idx[row]], softplus(theta[idx[row]]), re-drive row col[row] as int bits (col null: -1), bias[row] or 0}
+    // (see FwdEpi::info).  TRANSPOSE: out[j][a] = w[a][j] for a < rows, 0 up to ma (the read-out weights).
+    long long n = 0;                  // positions, rows or segments, or n_dn * ma
+    const int *idx = nullptr, *col = nullptr;
+    const int4* seg = nullptr;
+    void* out = nullptr;
+    long long w = 0;                  // offset of the weights (RECORDS: of the bias; -1: none)
+    int rows = 0, cols = 0, ma = 0;   // TRANSPOSE: n_act, n_dn, readout_pad(n_act)
 };
-constexpr int PACK_JOBS = 4;
-hipError_t launch_pack_n(const PackJob* jobs, int n, hipStream_t st, bool bf16w = false);
+// the blocks a job takes
+long long derive_blocks(const DeriveJob& j);
+// Jobs [j0, j0 + n) of the table at `jobs` (device memory); first (device): each job's first block, counted from job 0;
+// b0, blocks: the first block and the number of blocks of the range.  set: the weights' set; gain, theta: its arrays.
+// bf16w: pair weights rounded to bfloat16 (nearest even), as the float32 of that value
+hipError_t launch_derive(const DeriveJob* jobs, const int* first, int njobs, long long b0, long long blocks,
+                         const float* set, const float* gain, const float* theta, bool bf16w, hipStream_t st);
 // src_rows / gz_rows: rows of the gathered state (a gather of a row outside it reads zeros).  src_fires: the source
 // layer's firing bitmaps (launch_fires_pack; fires_ld(src_rows) words per tile; tiled states only), or nullptr
 // (a tiled launch that fwd_deep names, without bitmaps, takes k_fwd_deep)
@@ -194,20 +206,17 @@ hipError_t launch_bwd_lds(const Plan& p, const int2* wlds, const int2* cw, const
                           const int* hot_rows, int hot, const float* hsrc, Lay lhs, float* gwpart, long long gw_ld,
                           const BwdEpi& epi, float* part, Lay lp, int T, int S, hipStream_t st);
 hipError_t launch_obs_in(const float* obs, float* x, int obs_dim, int B, hipStream_t st);
-// the read-out on the matrix cores (readout.hip): owT, n_dn x readout_pad(n_act) floats of scratch for the
-// transposed weights; hK float32 tiles of 32 or (bf16_states) bfloat16 tiles of 64
+// the read-out on the matrix cores (readout.hip): owT, the weights transposed, n_dn x
+// readout_pad(n_act); hK float32 tiles of 32 or (bf16_states) bfloat16 tiles of 64
 int readout_pad(int n_act);
-hipError_t launch_owT(const float* ow, int n_act, int n_dn, float* owT, hipStream_t st);
 hipError_t launch_readout_bwd_w_mfma(const float* dl, const void* hK, bool bf16_states, int rows, const int* dn,
                                      int n_dn, int n_act, float* gow_part, float* gob_part, int B, hipStream_t st);
 hipError_t launch_readout_bwd_h_mfma(const float* dl, const float* owT, const int* dn_inv, int n_act, int rows,
                                      const BwdEpi& epi, int B, hipStream_t st);
 // lpart: RO_SPLIT x B x n_act floats of scratch (the sums over each split of the read-out rows)
 constexpr int RO_SPLIT = 8;
-// (owT_current: owT already holds ow transposed, so the transpose is not launched again)
-hipError_t launch_logits_mfma(const void* hK, bool bf16_states, int rows, const int* dn, int n_dn, const float* ow,
-                              const float* ob, int n_act, float* owT, float* lpart, float* logits, int B,
-                              hipStream_t st, bool owT_current = false);
+hipError_t launch_logits_mfma(const void* hK, bool bf16_states, int rows, const int* dn, int n_dn, const float* ob,
+                              int n_act, const float* owT, float* lpart, float* logits, int B, hipStream_t st);
 // the read-out weights' gradient partials come per chunk of RO_CHUNK_S samples: readout_chunks(B) of them
 constexpr int RO_CHUNK_S = 128;
 int readout_chunks(int B);
@@ -300,18 +309,4 @@ struct AdamSeg {
 hipError_t launch_adam(float* P, const float* G, float* M, float* V, float* EMA, const AdamSeg& s, float c1, float c2,
                        const float* gs_dev, float gs, float decay, hipStream_t st);
 hipError_t launch_export(const float* src, Lay ls, float* dst, int rows, int B, hipStream_t st);
-// per row of a layer its record {gain[nid], softplus(theta[nid]), re-drive row, 0} (see FwdEpi::info), for up to
-// ROW_JOBS layers in one launch
-struct RowJob {
-    const int *nid = nullptr, *drow = nullptr;
-    float4* info = nullptr;
-    int rows = 0;
-    // non-null: the records in the order of a row plan's segments instead (rows = the plan's segments, row = seg.x),
-    // so that a wave's 8 rows read one 128-byte line (FwdEpi::sinfo)
-    const int4* seg = nullptr;
-    const float* bias = nullptr;      // non-null: the records' fourth field is bias[row] (the plug's rows), else 0
-};
-constexpr int ROW_JOBS = 8;
-hipError_t launch_rowinfo_n(const RowJob* jobs, int n, const float* gain, const float* theta, hipStream_t st);
-
 }  // namespace fg

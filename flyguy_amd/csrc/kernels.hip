@@ -52,24 +52,67 @@ static bool fill_table(JobTable<J, N>& t, const J* jobs, int n, Elems elems, lon
     return nb <= 0xFFFFFFFFLL;
 }
 
-// the (source, weight) pair of every plan position, from the current weights; BF16W: the weight rounded to bfloat16
-// (nearest even), kept as the float32 of that value (low 16 bits zero)
-template <bool BF16W>
-__global__ __launch_bounds__(WG) void k_pack(JobTable<PackJob, PACK_JOBS> t) {
-    long long b0;
-    const PackJob J = job_of(t, blockIdx.x, b0);
-    const long long p = ((long long)blockIdx.x - b0) * WG + threadIdx.x;
-    if (p >= J.n) return;
-    const int i = J.pidx[p];
-    float v = i >= 0 ? J.w[i] : 0.f;
-    if (BF16W) v = (float)(__bf16)v;
-    if (J.pb == 6) {                            // (Plan::pb) the weight plane, then the source plane of the step
-        unsigned char* blk = reinterpret_cast<unsigned char*>(J.cw) + (size_t)(p >> 6) * 384;
+// the (source, weight) pair of every plan position, from the given weights
+__global__ __launch_bounds__(WG) void k_pack(const int* __restrict__ pcol, const int* __restrict__ pidx,
+                                             const float* __restrict__ w, int2* __restrict__ cw, long long n, int pb) {
+    const long long p = (long long)blockIdx.x * WG + threadIdx.x;
+    if (p >= n) return;
+    const int i = pidx[p];
+    const float v = i >= 0 ? w[i] : 0.f;
+    if (pb == 6) {                              // (Plan::pb) the weight plane, then the source plane of the step
+        unsigned char* blk = reinterpret_cast<unsigned char*>(cw) + (size_t)(p >> 6) * 384;
         reinterpret_cast<float*>(blk)[p & 63] = v;
-        reinterpret_cast<unsigned short*>(blk + 256)[p & 63] = i >= 0 ? (unsigned short)J.pcol[p] : (unsigned short)0xFFFF;
+        reinterpret_cast<unsigned short*>(blk + 256)[p & 63] = i >= 0 ? (unsigned short)pcol[p] : (unsigned short)0xFFFF;
         return;
     }
-    J.cw[p] = i >= 0 ? make_int2(J.pcol[p], __float_as_int(v)) : make_int2(NO_ROW, 0);
+    cw[p] = i >= 0 ? make_int2(pcol[p], __float_as_int(v)) : make_int2(NO_ROW, 0);
+}
+
+// Every table of a pass that follows the weights, in one launch (kernels.h, DeriveJob): a teaching step makes them all
+// anew, and apart they were six launches of 4 to 35 us.  A wave finds its job among the table's first blocks with a
+// ballot.  The pairs' cost is the gather of the strengths in the transposed plans' order (12 MB, one 4-byte value a
+// line); four (two) gathers per thread are in flight, and 6-byte pairs rewrite their weight planes only.
+constexpr int DERIVE_PER[] = {2, 4, 1, 1};      // elements per thread of each kind
+template <bool BF16W>
+__global__ __launch_bounds__(WG) void k_derive(const DeriveJob* __restrict__ jobs, const int* __restrict__ first,
+                                               int njobs, int b0, const float* __restrict__ set,
+                                               const float* __restrict__ gain, const float* __restrict__ theta) {
+    const int b = b0 + (int)blockIdx.x, lane = threadIdx.x & 63;
+    int k = -1;
+    for (int i = lane; i - lane < njobs; i += 64) k += __popcll(__ballot(i < njobs && first[i] <= b));
+    k = __builtin_amdgcn_readfirstlane(k);
+    const DeriveJob& J = jobs[k];
+    const int kind = J.kind;
+    const long long t = (long long)(b - first[k]) * WG + threadIdx.x;
+    auto weight = [&](int i) {
+        float v = i >= 0 ? set[J.w + i] : 0.f;
+        if (BF16W) v = (float)(__bf16)v;
+        return v;
+    };
+    if (kind == DeriveJob::PAIRS8) {
+        if (2 * t >= J.n) return;
+        const int2 i = reinterpret_cast<const int2*>(J.idx)[t], c = reinterpret_cast<const int2*>(J.col)[t];
+        const float x = weight(i.x), y = weight(i.y);
+        reinterpret_cast<int4*>(J.out)[t] = make_int4(i.x >= 0 ? c.x : NO_ROW, __float_as_int(x), i.y >= 0 ? c.y : NO_ROW,
+                                                      __float_as_int(y));
+    } else if (kind == DeriveJob::WEIGHTS6) {
+        if (4 * t >= J.n) return;
+        const int4 i = reinterpret_cast<const int4*>(J.idx)[t];
+        const float x = weight(i.x), y = weight(i.y), z = weight(i.z), w = weight(i.w);
+        // (a step's 64 weights, 16 threads, at the start of its 384 bytes)
+        reinterpret_cast<float4*>(reinterpret_cast<unsigned char*>(J.out) + (size_t)(t >> 4) * 384)[t & 15] =
+            make_float4(x, y, z, w);
+    } else if (kind == DeriveJob::RECORDS) {
+        if (t >= J.n) return;
+        const int row = J.seg ? J.seg[t].x : (int)t, n = J.idx[row];
+        reinterpret_cast<float4*>(J.out)[t] = make_float4(gain[n], softplus_f(theta[n]),
+                                                          __int_as_float(J.col ? J.col[row] : -1),
+                                                          J.w >= 0 ? set[J.w + row] : 0.f);
+    } else {
+        if (t >= J.n) return;
+        const int j = (int)(t / J.ma), a = (int)(t % J.ma);
+        reinterpret_cast<float*>(J.out)[t] = a < J.rows ? set[J.w + (size_t)a * J.cols + j] : 0.f;
+    }
 }
 
 // ------------------------------------------------------------------------------------------------ forward
@@ -1265,19 +1308,6 @@ __global__ void k_adam(float* __restrict__ P, const float* __restrict__ G, float
     EMA[i] = fmaf(decay, EMA[i], (1.f - decay) * pi);
 }
 
-// per row of a layer: {gain[nid], softplus(theta[nid]), re-drive row (int bits, -1 none), bias of the row or 0}
-__global__ __launch_bounds__(WG) void k_rowinfo(JobTable<RowJob, ROW_JOBS> t, const float* __restrict__ gain,
-                                                const float* __restrict__ theta) {
-    long long b0;
-    const RowJob J = job_of(t, blockIdx.x, b0);
-    const long long r = ((long long)blockIdx.x - b0) * WG + threadIdx.x;
-    if (r >= J.rows) return;
-    const int row = J.seg ? J.seg[r].x : (int)r;
-    const int n = J.nid[row];
-    J.info[r] = make_float4(gain[n], softplus_f(theta[n]), __int_as_float(J.drow ? J.drow[row] : -1),
-                            J.bias ? J.bias[row] : 0.f);
-}
-
 // a state tensor (tiled) -> [rows][B] (tests and diagnostics)
 __global__ void k_export(const float* __restrict__ src, Lay ls, float* __restrict__ dst, int rows, int B) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1289,26 +1319,31 @@ __global__ void k_export(const float* __restrict__ src, Lay ls, float* __restric
 // ------------------------------------------------------------------------------------------------ launchers
 static inline unsigned blocks(long long n, int per = WG) { return (unsigned)((n + per - 1) / per); }
 
-hipError_t launch_pack_n(const PackJob* jobs, int n, hipStream_t st, bool bf16w) {
-    JobTable<PackJob, PACK_JOBS> t;
-    long long nb;
-    if (!fill_table(t, jobs, n, [](const PackJob& j) { return j.n; }, nb)) return hipErrorInvalidValue;
-    for (int k = 0; k < t.n; ++k)
-        if (!t.j[k].pcol || !t.j[k].pidx || !t.j[k].w || !t.j[k].cw || (t.j[k].pb != 8 && t.j[k].pb != 6) ||
-            (t.j[k].pb == 6 && t.j[k].n % 64))
-            return hipErrorInvalidValue;
-    if (nb == 0) return hipSuccess;
-    if (bf16w)
-        k_pack<true><<<(unsigned)nb, WG, 0, st>>>(t);
-    else
-        k_pack<false><<<(unsigned)nb, WG, 0, st>>>(t);
+hipError_t launch_pack(const int* pcol, const int* pidx, const float* w, int2* cw, long long npos, hipStream_t st,
+                       int pb) {
+    if (npos <= 0) return hipSuccess;
+    if (!pcol || !pidx || !w || !cw || (pb != 8 && pb != 6) || (pb == 6 && npos % 64)) return hipErrorInvalidValue;
+    const long long nb = (npos + WG - 1) / WG;
+    if (nb > 0xFFFFFFFFLL) return hipErrorInvalidValue;
+    k_pack<<<(unsigned)nb, WG, 0, st>>>(pcol, pidx, w, cw, npos, pb);
     return hipGetLastError();
 }
 
-hipError_t launch_pack(const int* pcol, const int* pidx, const float* w, int2* cw, long long npos, hipStream_t st,
-                       bool bf16w) {
-    const PackJob j{pcol, pidx, w, cw, npos};
-    return launch_pack_n(&j, 1, st, bf16w);
+long long derive_blocks(const DeriveJob& j) {
+    const long long per = (long long)WG * DERIVE_PER[j.kind];
+    return (j.n + per - 1) / per;
+}
+
+hipError_t launch_derive(const DeriveJob* jobs, const int* first, int njobs, long long b0, long long blocks,
+                         const float* set, const float* gain, const float* theta, bool bf16w, hipStream_t st) {
+    if (blocks <= 0) return hipSuccess;
+    if (!jobs || !first || njobs <= 0 || b0 < 0 || b0 + blocks > 0x7FFFFFFFLL || !set || !gain || !theta)
+        return hipErrorInvalidValue;
+    if (bf16w)
+        k_derive<true><<<(unsigned)blocks, WG, 0, st>>>(jobs, first, njobs, (int)b0, set, gain, theta);
+    else
+        k_derive<false><<<(unsigned)blocks, WG, 0, st>>>(jobs, first, njobs, (int)b0, set, gain, theta);
+    return hipGetLastError();
 }
 
 hipError_t launch_fwd(const Plan& p, const int2* cw, const float* src, Lay ls, int src_rows, const FwdEpi& epi,
@@ -1612,17 +1647,6 @@ hipError_t launch_adam(float* P, const float* G, float* M, float* V, float* EMA,
                        const float* gs_dev, float gs, float decay, hipStream_t st) {
     (void)gs_dev;
     k_adam<<<blocks(s.off[7]), WG, 0, st>>>(P, G, M, V, EMA, s, c1, c2, gs, decay);
-    return hipGetLastError();
-}
-
-hipError_t launch_rowinfo_n(const RowJob* jobs, int n, const float* gain, const float* theta, hipStream_t st) {
-    JobTable<RowJob, ROW_JOBS> t;
-    long long nb;
-    if (!fill_table(t, jobs, n, [](const RowJob& j) { return (long long)j.rows; }, nb)) return hipErrorInvalidValue;
-    for (int k = 0; k < t.n; ++k)
-        if (!t.j[k].nid || !t.j[k].info) return hipErrorInvalidValue;
-    if (nb == 0) return hipSuccess;
-    k_rowinfo<<<(unsigned)nb, WG, 0, st>>>(t, gain, theta);
     return hipGetLastError();
 }
 

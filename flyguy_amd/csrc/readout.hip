@@ -9,14 +9,6 @@
 
 namespace fg {
 
-// owT[j][a] = ow[a][j] for a < n_act, 0 up to ma (a multiple of 32)
-__global__ void k_owT(const float* __restrict__ ow, int n_act, int n_dn, int ma, float* __restrict__ owT) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)n_dn * ma) return;
-    const int j = (int)(i / ma), a = (int)(i % ma);
-    owT[i] = a < n_act ? ow[(size_t)a * n_dn + j] : 0.f;
-}
-
 template <bool BF16S>
 __device__ __forceinline__ float state_at(const void* hK, size_t i) {
     if (BF16S) return __uint_as_float((unsigned)reinterpret_cast<const unsigned short*>(hK)[i] << 16);
@@ -166,13 +158,6 @@ __global__ __launch_bounds__(WG) void k_readout_bwd_w_mfma(const float* __restri
 
 int readout_pad(int n_act) { return (n_act + 31) / 32 * 32; }
 
-hipError_t launch_owT(const float* ow, int n_act, int n_dn, float* owT, hipStream_t st) {
-    const int ma = readout_pad(n_act);
-    const long long n = (long long)n_dn * ma;
-    k_owT<<<(unsigned)((n + WG - 1) / WG), WG, 0, st>>>(ow, n_act, n_dn, ma, owT);
-    return hipGetLastError();
-}
-
 hipError_t launch_readout_bwd_w_mfma(const float* dl, const void* hK, bool bf16_states, int rows, const int* dn,
                                      int n_dn, int n_act, float* gow_part, float* gob_part, int B, hipStream_t st) {
     if (readout_pad(n_act) > 32 * RO_MAXB || n_act > WG) return hipErrorInvalidValue;
@@ -184,24 +169,20 @@ hipError_t launch_readout_bwd_w_mfma(const float* dl, const void* hK, bool bf16_
     return hipGetLastError();
 }
 
-hipError_t launch_logits_mfma(const void* hK, bool bf16_states, int rows, const int* dn, int n_dn, const float* ow,
-                              const float* ob, int n_act, float* owT, float* lpart, float* logits, int B,
-                              hipStream_t st, bool owT_current) {
+hipError_t launch_logits_mfma(const void* hK, bool bf16_states, int rows, const int* dn, int n_dn, const float* ob,
+                              int n_act, const float* owT, float* lpart, float* logits, int B, hipStream_t st) {
     const int ma = readout_pad(n_act);
     if (ma > 32 * RO_MAXB || B % 32 != 0) return hipErrorInvalidValue;
     const size_t sm = (size_t)((n_dn + 3) & ~3) * sizeof(int) + (size_t)RO_WAVES * 32 * 33 * sizeof(float);
     if (sm > 64 * 1024) return hipErrorInvalidValue;
-    const long long n = (long long)n_dn * ma;
-    if (!owT_current) k_owT<<<(unsigned)((n + WG - 1) / WG), WG, 0, st>>>(ow, n_act, n_dn, ma, owT);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || B == 0) return e;
+    if (B == 0) return hipSuccess;
     const dim3 grid((unsigned)(B / 32), RO_SPLIT);
     const unsigned threads = 64 * RO_WAVES;
     if (bf16_states)
         k_logits_mfma<true><<<grid, threads, sm, st>>>(hK, rows, TW16, dn, n_dn, owT, ma, n_act, lpart);
     else
         k_logits_mfma<false><<<grid, threads, sm, st>>>(hK, rows, TW, dn, n_dn, owT, ma, n_act, lpart);
-    e = hipGetLastError();
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const long long nl = (long long)B * n_act;
     k_logits_sum<<<(unsigned)((nl + WG - 1) / WG), WG, 0, st>>>(lpart, ob, n_act, nl, logits);
