@@ -111,6 +111,7 @@ struct Core {
     int plug_lds = -1;               // the plug staged in LDS: -1 by batch size, 0 never, S > 0 with S workgroups per tile
     int bwd_lds = -1;                // k_bwd_lds for the hops that have it: -1 from BWD_LDS_MIN_TILES tiles up, 0 never,
                                      //   1 at every batch (FLYGUY_BWD_LDS)
+    int dev = -1;                    // the device the handle was made on
     int cus = 0;                     // the device's CUs (k_bwd_lds takes one workgroup per CU)
     // What the derived tables were made from.  wver[set] counts the writes to the weights (set 0) and to the running
     // average (set 1): fc_copy into the handle, an Adam step, the trainer's host-side edits.  A table made from a
@@ -122,6 +123,9 @@ struct Core {
         bool same(int s, unsigned long long v) const { return set == s && ver == v; }
     };
     unsigned long long wver[2] = {1, 1};
+    // Whether the gradient entries that no backward writes (neurons and strengths out of play, the arrays' padding) are
+    // zero: until a gradient is copied in.  A step whose backward stores every other entry (fresh) clears nothing then.
+    bool grad_rest_zero = true;
     // The tables in the order of their jobs (DeriveJob), each group a run of blocks: group g's are [dblock[g], dblock[g + 1])
     enum Table { T_FPAIRS = 0, T_INFO = 1, T_OWT = 2, T_TPAIRS = 3, T_COUNT = 4 };
     Stamp made[T_COUNT];
@@ -181,13 +185,15 @@ bool prof_collect(Core& c);
 // logits [B][n_act]
 bool forward(Core& c, const float* obs, int B, float* logits, int set);
 // backward of the last forward (through SET_P) from dlogits [B][n_act]: gradients ADDED to the SET_G arrays
-// fresh: the gradient arrays are zero and this backward is the only one adding to them (a teaching step), so the
-// first sum into each entry is stored instead of added (no read of the entry)
+// fresh: the gradient starts from zero and this backward is the only one adding to it (a teaching step), so the first
+// sum into each entry is stored instead of added (no read of the entry)
 bool backward(Core& c, const float* dlogits, int B, bool fresh = false);
 // Makes the tables that passes derive from the weights and that are not current: the forward's (from `set`) and / or
 // the backward's (from the weights, so with bwd the set is SET_P).  forward() and backward() call it for their own; a
 // step that runs both calls it for both first, in one launch.
 bool derive(Core& c, int set, bool fwd, bool bwd);
+// Ahead of a fresh backward: clears the gradient, unless what that backward does not store is zero already
+bool clear_for_fresh(Core& c);
 float grad_norm(Core& c);
 // Adam + running average over all seven arrays; lr for W, lr_neuron for gain / theta, lr_plug for the rest
 float step(Core& c, float lr, float lr_neuron, float lr_plug, float max_norm, float ema);

@@ -540,8 +540,8 @@ Core* build(const unsigned char* bytes, long long len, int max_batch, int prec) 
     const int lds_cap = c->bwd_lds == 0 ? 0 : (prec ? bwd_lds_rows16() : bwd_lds_rows());
     {
         int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        if (hipGetDevice(&dev) == hipSuccess) c->dev = dev;
+        if (c->dev < 0 || hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             c->cus = 0;
     }
     for (int k = 0; k < K; ++k) {
@@ -1132,6 +1132,14 @@ static bool backward16(Core& c, const float* dlogits, int B, bool fresh) {
     return true;
 }
 
+bool clear_for_fresh(Core& c) {
+    if (c.grad_rest_zero) return true;
+    Timed t(c, ST_ZERO);
+    FG_CHECK(launch_fill(c.arr(SET_G, 0), 0.f, c.PT, c.st), false);
+    c.grad_rest_zero = true;
+    return true;
+}
+
 float grad_norm(Core& c) {
     if (launch_sumsq(c.arr(SET_G, 0), c.PT, c.red, c.nrm, c.st) != hipSuccess) { set_error("grad norm launch"); return -1.f; }
     float ss = 0.f;
@@ -1165,6 +1173,21 @@ float step(Core& c, float lr, float lr_neuron, float lr_plug, float max_norm, fl
 }  // namespace fg
 
 using namespace fg;
+
+// whether a kernel on the handle's stream may read and write `bytes` at p: memory of the handle's device, which is the
+// current one, inside one allocation
+static bool on_device(const Core& c, const void* p, size_t bytes) {
+    hipPointerAttribute_t a{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    int dev = -1;
+    const bool ok = hipGetDevice(&dev) == hipSuccess && dev == c.dev && hipPointerGetAttributes(&a, p) == hipSuccess &&
+                    a.type == hipMemoryTypeDevice && a.device == dev &&
+                    hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) == hipSuccess &&
+                    (const char*)p + bytes <= (const char*)base + size;
+    if (!ok) (void)hipGetLastError();
+    return ok;
+}
 
 // ================================================================================================ C-ABI
 extern "C" {
@@ -1216,13 +1239,21 @@ void fc_sizes(void* h, long long* out) {
 void fc_copy(void* h, int which, int to_core, float** ptrs) {
     Core* c = (Core*)h;
     if (!c || !ptrs || which < 0 || which > 4) { set_error("fc_copy: bad argument"); return; }
+    CopyJobs jobs;
     for (int i = 0; i < 7; ++i) {
         if (!ptrs[i]) continue;
         float* lib = c->arr(which, i);
-        FG_CHECK(hipMemcpyAsync(to_core ? lib : ptrs[i], to_core ? ptrs[i] : lib, c->psize[i] * 4, hipMemcpyDeviceToDevice,
-                                c->st), );
-        if (to_core) c->weights_written(which);
+        if (to_core) {
+            c->weights_written(which);
+            if (which == SET_G) c->grad_rest_zero = false;
+        }
+        if (on_device(*c, ptrs[i], (size_t)c->psize[i] * 4))
+            jobs.add(to_core ? ptrs[i] : lib, to_core ? lib : ptrs[i], c->psize[i]);
+        else                                    // (memory of another device or the host, or too short: the runtime's copy)
+            FG_CHECK(hipMemcpyAsync(to_core ? lib : ptrs[i], to_core ? ptrs[i] : lib, c->psize[i] * 4,
+                                    hipMemcpyDeviceToDevice, c->st), );
     }
+    FG_CHECK(launch_copy(jobs, c->st), );
     FG_CHECK(hipStreamSynchronize(c->st), );
 }
 
@@ -1237,6 +1268,7 @@ void fc_zero_grad(void* h) {
     Core* c = (Core*)h;
     if (!c) { set_error("null handle"); return; }
     FG_CHECK(launch_fill(c->arr(SET_G, 0), 0.f, c->PT, c->st), );
+    c->grad_rest_zero = true;
 }
 
 void fc_backward(void* h, const float* dlogits, int B) {
@@ -1279,13 +1311,12 @@ float fc_teach_step(void* h, const float* obs, const float* teacher, int B, floa
     Core* c = (Core*)h;
     if (!check_batch(c, B)) return -1.f;
     if (!obs || !teacher) { set_error("fc_teach_step: null pointer"); return -1.f; }
-    { Timed t(*c, ST_ZERO); FG_CHECK(launch_fill(c->arr(SET_G, 0), 0.f, c->PT, c->st), -1.f); }
-    if (!derive(*c, SET_P, true, true) || !forward(*c, obs, B, c->lg, SET_P)) return -1.f;
+    if (!clear_for_fresh(*c) || !derive(*c, SET_P, true, true) || !forward(*c, obs, B, c->lg, SET_P)) return -1.f;
     {
         Timed t(*c, ST_LOSS);
         FG_CHECK(launch_loss(c->lg, teacher, c->dl, c->stats_part, stats ? stats : c->stats, c->n_act, B, it, c->st), -1.f);
     }
-    if (!backward(*c, c->dl, B, true)) return -1.f;          // (the gradient was cleared above)
+    if (!backward(*c, c->dl, B, true)) return -1.f;
     return step(*c, lr, lr_neuron, lr_plug, max_norm, ema);
 }
 

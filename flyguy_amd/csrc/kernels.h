@@ -301,6 +301,19 @@ hipError_t launch_readout_bwd_h16_mfma(const float* dl, const float* owT, const 
 hipError_t launch_loss(const float* lg, const float* tl, float* dl, float* stats_part, float* stats, int n_act, int B,
                        float it, hipStream_t st, bool accumulate = false);
 hipError_t launch_fill(float* p, float v, long long n, hipStream_t st);
+// up to 7 arrays of floats copied in one launch (source and destination: memory of the current device, apart)
+struct CopyJobs {
+    const float* src[7] = {};
+    float* dst[7] = {};
+    long long n[7] = {};
+    int count = 0;
+    void add(const float* s, float* d, long long m) {
+        src[count] = s;
+        dst[count] = d;
+        n[count++] = m;
+    }
+};
+hipError_t launch_copy(const CopyJobs& j, hipStream_t st);
 hipError_t launch_sumsq(const float* g, long long n, float* part, float* out, hipStream_t st);
 struct AdamSeg {
     long long off[8];

@@ -1198,6 +1198,7 @@ __global__ __launch_bounds__(256) void k_loss(const float* __restrict__ lg, cons
     __shared__ float red[2][4];
     const int b0 = blockIdx.x * LOSS_S, nb = min(LOSS_S, B - b0);
     const size_t base = (size_t)b0 * n_act;
+#pragma unroll 4
     for (int i = threadIdx.x; i < nb * n_act; i += 256) {
         S[i] = lg[base + i];
         Tt[i] = tl[base + i] * it;
@@ -1259,17 +1260,57 @@ __global__ __launch_bounds__(256) void k_loss(const float* __restrict__ lg, cons
         stats_part[2 * blockIdx.x + 1] = ((red[1][0] + red[1][1]) + red[1][2]) + red[1][3];
     }
 }
-__global__ void k_sum_pairs(const float* __restrict__ part, int n, float* __restrict__ out, int acc) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    float a = 0.f, b = 0.f;
-    for (int i = 0; i < n; ++i) { a += part[2 * i]; b += part[2 * i + 1]; }
-    out[0] = acc ? out[0] + a : a;
-    out[1] = acc ? out[1] + b : b;
+// the n values (of each of W arrays, interleaved) added in order by one thread, from LDS: the loads go out together.
+// Read one at a time, 128 pairs took 7 us and 512 took 32.
+constexpr int SUM_STAGE = 2048;                 // values staged at a time
+template <int W>
+__device__ __forceinline__ void ordered_sums(const float* __restrict__ part, int n, float (&s)[W]) {
+    __shared__ float v[SUM_STAGE];
+    for (int b = 0; b < n * W; b += SUM_STAGE) {
+        const int m = min(SUM_STAGE, n * W - b);
+        for (int i = threadIdx.x; i < m; i += WG) v[i] = part[b + i];
+        __syncthreads();
+        if (threadIdx.x == 0) {
+#pragma unroll 16
+            for (int i = 0; i < m; i += W)
+#pragma unroll
+                for (int k = 0; k < W; ++k) s[k] += v[i + k];
+        }
+        __syncthreads();
+    }
+}
+__global__ __launch_bounds__(WG) void k_sum_pairs(const float* __restrict__ part, int n, float* __restrict__ out, int acc) {
+    float s[2] = {0.f, 0.f};
+    ordered_sums<2>(part, n, s);
+    if (threadIdx.x != 0) return;
+    out[0] = acc ? out[0] + s[0] : s[0];
+    out[1] = acc ? out[1] + s[1] : s[1];
 }
 
 __global__ void k_fill(float* __restrict__ p, float v, long long n) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
+}
+
+// Array k of the jobs by the blocks (., k), 16 bytes a thread and turn where both ends are aligned for it.  Seven copies
+// of the runtime's, 4 to 6 us each, take 34 us for the benchmark network's arrays (14 MB); this launch 9 us.
+__global__ __launch_bounds__(WG) void k_copy(CopyJobs j) {
+    const int k = blockIdx.y;
+    const float* src = j.src[0];
+    float* dst = j.dst[0];
+    long long n = j.n[0];
+#pragma unroll
+    for (int i = 1; i < 7; ++i)
+        if (k == i) { src = j.src[i]; dst = j.dst[i]; n = j.n[i]; }
+    const long long step = (long long)gridDim.x * WG;
+    long long i = (long long)blockIdx.x * WG + threadIdx.x, done = 0;
+    if ((((size_t)src | (size_t)dst) & 15) == 0) {
+        const float4* s4 = reinterpret_cast<const float4*>(src);
+        float4* d4 = reinterpret_cast<float4*>(dst);
+        for (long long q = i; q < n / 4; q += step) d4[q] = s4[q];
+        done = n / 4 * 4;
+    }
+    for (i += done; i < n; i += step) dst[i] = src[i];
 }
 
 __global__ __launch_bounds__(WG) void k_sumsq(const float* __restrict__ g, long long n, float* __restrict__ part) {
@@ -1284,11 +1325,10 @@ __global__ __launch_bounds__(WG) void k_sumsq(const float* __restrict__ g, long 
     }
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
-__global__ void k_sum(const float* __restrict__ part, int n, float* __restrict__ out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    float a = 0.f;
-    for (int i = 0; i < n; ++i) a += part[i];
-    out[0] = a;
+__global__ __launch_bounds__(WG) void k_sum(const float* __restrict__ part, int n, float* __restrict__ out) {
+    float s[1] = {0.f};
+    ordered_sums<1>(part, n, s);
+    if (threadIdx.x == 0) out[0] = s[0];
 }
 
 // one Adam step with a running average of the weights over all seven arrays (flyguy_train.cu:194-203)
@@ -1624,7 +1664,7 @@ hipError_t launch_loss(const float* lg, const float* tl, float* dl, float* stats
     k_loss<<<nb, 256, (size_t)2 * LOSS_S * n_act * sizeof(float), st>>>(lg, tl, dl, stats_part, n_act, B, it);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_sum_pairs<<<1, 64, 0, st>>>(stats_part, (int)nb, stats, accumulate ? 1 : 0);
+    k_sum_pairs<<<1, WG, 0, st>>>(stats_part, (int)nb, stats, accumulate ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -1634,12 +1674,21 @@ hipError_t launch_fill(float* p, float v, long long n, hipStream_t st) {
     return hipGetLastError();
 }
 
+hipError_t launch_copy(const CopyJobs& j, hipStream_t st) {
+    long long most = 0;
+    for (int k = 0; k < j.count; ++k) most = std::max(most, j.n[k]);
+    if (most <= 0) return hipSuccess;
+    const unsigned nb = (unsigned)std::min<long long>((most + 4 * WG - 1) / (4 * WG), 2048);
+    k_copy<<<dim3(nb, (unsigned)j.count), WG, 0, st>>>(j);
+    return hipGetLastError();
+}
+
 hipError_t launch_sumsq(const float* g, long long n, float* part, float* out, hipStream_t st) {
     const int nb = 1024;
     k_sumsq<<<nb, WG, 0, st>>>(g, n, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_sum<<<1, 64, 0, st>>>(part, nb, out);
+    k_sum<<<1, WG, 0, st>>>(part, nb, out);
     return hipGetLastError();
 }
 

@@ -94,9 +94,28 @@ __global__ __launch_bounds__(WG) void k_logits_sum(const float* __restrict__ lpa
     logits[i] = ob[i % n_act] + v;
 }
 
+// out[a] = sum over samples b0 .. b1 of dl[b][a], in sample order, 16 loads in flight (an action per thread).  One after
+// another, behind a workgroup's products, they took 14 of the kernel's 22 us at B=512.
+__device__ __forceinline__ void readout_bias_chunk(const float* __restrict__ dl, int n_act, int b0, int b1,
+                                                   float* __restrict__ out) {
+    const int a = threadIdx.x;
+    if (a >= n_act) return;
+    float s = 0.f;
+    int b = b0;
+    for (; b + 16 <= b1; b += 16) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = dl[(size_t)(b + u) * n_act + a];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s += v[u];
+    }
+    for (; b < b1; ++b) s += dl[(size_t)b * n_act + a];
+    out[a] = s;
+}
+
 // The read-out weights' gradient per chunk of RO_CHUNK_S samples (flyguy_train.cu:125-135):
 //   gow_part[chunk][a][j] = sum_b dl[b][a] hK[dn[j]][b],  gob_part[chunk][a] = sum_b dl[b][a]  (b in the chunk)
-// Grid (n_dn / 32 blocks of read-out rows, chunks), 256 threads: the 4 waves each take a quarter of the chunk's
+// Grid (n_dn / 32 blocks of read-out rows and one for the bias, chunks), 256 threads: the 4 waves each take a quarter of the chunk's
 // samples for every block of 32 actions (M = actions, N = read-out rows, K = samples); partials added through LDS in
 // wave order.  Short chunks keep each wave's chain of dependent loads short (4 steps of 8 samples).
 template <bool BF16S>
@@ -106,6 +125,11 @@ __global__ __launch_bounds__(WG) void k_readout_bwd_w_mfma(const float* __restri
                                                            float* __restrict__ gob_part) {
     __shared__ float part[4 * 32 * 33];
     const int j0 = blockIdx.x * 32, chunk = blockIdx.y;
+    if (j0 >= n_dn) {                           // the last block of a chunk: the bias's sums
+        readout_bias_chunk(dl, n_act, chunk * RO_CHUNK_S, min(B, (chunk + 1) * RO_CHUNK_S),
+                           gob_part + (size_t)chunk * n_act);
+        return;
+    }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 31, kk = lane >> 5;
     const int nb = (n_act + 31) / 32;
     const int row = j0 + i < n_dn ? dn[j0 + i] : -1;
@@ -148,12 +172,6 @@ __global__ __launch_bounds__(WG) void k_readout_bwd_w_mfma(const float* __restri
         }
         __syncthreads();
     }
-    if (blockIdx.x == 0 && (int)threadIdx.x < n_act) {
-        float sb = 0.f;
-        for (int b = min(B, chunk * RO_CHUNK_S); b < min(B, (chunk + 1) * RO_CHUNK_S); ++b)
-            sb += dl[(size_t)b * n_act + threadIdx.x];
-        gob_part[(size_t)chunk * n_act + threadIdx.x] = sb;
-    }
 }
 
 int readout_pad(int n_act) { return (n_act + 31) / 32 * 32; }
@@ -161,7 +179,7 @@ int readout_pad(int n_act) { return (n_act + 31) / 32 * 32; }
 hipError_t launch_readout_bwd_w_mfma(const float* dl, const void* hK, bool bf16_states, int rows, const int* dn,
                                      int n_dn, int n_act, float* gow_part, float* gob_part, int B, hipStream_t st) {
     if (readout_pad(n_act) > 32 * RO_MAXB || n_act > WG) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((n_dn + 31) / 32), (unsigned)readout_chunks(B));
+    const dim3 grid((unsigned)((n_dn + 31) / 32 + 1), (unsigned)readout_chunks(B));
     if (bf16_states)
         k_readout_bwd_w_mfma<true><<<grid, WG, 0, st>>>(dl, hK, rows, TW16, dn, n_dn, n_act, B, gow_part, gob_part);
     else

@@ -888,10 +888,9 @@ static void rates_at(long long step, float lr, float lr_neuron, float lr_plug, f
 
 // one forward + loss + backward of a staged batch; the loss sums ADDED to stats
 static bool learn_from(Core& c, const float* obs, const float* tl, int B, float it, float* stats) {
-    FG_CHECK(launch_fill(c.arr(SET_G, 0), 0.f, c.PT, c.st), false);
-    if (!derive(c, SET_P, true, true) || !forward(c, obs, B, c.lg, SET_P)) return false;
+    if (!clear_for_fresh(c) || !derive(c, SET_P, true, true) || !forward(c, obs, B, c.lg, SET_P)) return false;
     FG_CHECK(launch_loss(c.lg, tl, c.dl, c.stats_part, stats, c.n_act, B, it, c.st, true), false);
-    return backward(c, c.dl, B, true);                      // (the gradient was cleared above)
+    return backward(c, c.dl, B, true);
 }
 
 typedef std::unique_ptr<Core, void (*)(Core*)> CoreP;
