@@ -18,6 +18,18 @@ template <> struct Bits16<F16> {
     static __device__ __forceinline__ unsigned from(float x) {   // round to nearest even
         return (unsigned)__builtin_bit_cast(unsigned short, (_Float16)x);
     }
+    // lo(w) a + c and hi(w) a + c in one instruction, rounded once, as fmaf of the widened value.  Written out because
+    // the compiler widens a value that two sums use once, with an instruction of its own.
+    static __device__ __forceinline__ float fma_lo(unsigned w, float a, float c) {
+        float r;
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(a), "v"(c));
+        return r;
+    }
+    static __device__ __forceinline__ float fma_hi(unsigned w, float a, float c) {
+        float r;
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(a), "v"(c));
+        return r;
+    }
 };
 template <> struct Bits16<BF16> {
     static __device__ __forceinline__ float lo(unsigned w) { return __uint_as_float(w << 16); }

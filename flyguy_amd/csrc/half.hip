@@ -41,11 +41,32 @@ __global__ void k_to16(const float* __restrict__ x, int rows, int B, const float
     *reinterpret_cast<u32x4*>(dst + (size_t)rt * TW16 + sub * 8) = o;
 }
 
-// *out = max(*out, max |x|) over non-negative floats (whose order is that of their bit patterns)
+// *out = max(*out, max |x|) over non-negative floats (whose order is that of their bit patterns).  Bound by HBM: four
+// 16-byte loads in flight a thread where x is aligned for them (618 MB, hop 2's gradient at B=4096: 281 us with one
+// 4-byte load a turn, now 126 us).
 __global__ __launch_bounds__(WG) void k_absmax(const float* __restrict__ x, long long n, unsigned* __restrict__ out) {
     __shared__ float red[WG / 64];
     float m = 0.f;
-    for (long long i = (long long)blockIdx.x * WG + threadIdx.x; i < n; i += (long long)gridDim.x * WG) m = fmaxf(m, fabsf(x[i]));
+    const long long i0 = (long long)blockIdx.x * WG + threadIdx.x, step = (long long)gridDim.x * WG;
+    long long done = 0;
+    if (((size_t)x & 15) == 0) {
+        const float4* x4 = reinterpret_cast<const float4*>(x);
+        const long long n4 = n / 4;
+        auto take = [&](const float4& v) {
+            m = fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+        };
+        long long i = i0;
+        for (; i + 3 * step < n4; i += 4 * step) {
+            const float4 a = x4[i], b = x4[i + step], c = x4[i + 2 * step], d = x4[i + 3 * step];
+            take(a);
+            take(b);
+            take(c);
+            take(d);
+        }
+        for (; i < n4; i += step) take(x4[i]);
+        done = 4 * n4;
+    }
+    for (long long i = done + i0; i < n; i += step) m = fmaxf(m, fabsf(x[i]));
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -56,9 +77,18 @@ __global__ __launch_bounds__(WG) void k_absmax(const float* __restrict__ x, long
     }
 }
 
+// a lane's 8 samples to the row-major output, past the L2: a later kernel reads them, and they should not push out the
+// slab being gathered
+__device__ __forceinline__ void store8_stream(float* dst, const float (&a)[8]) {
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    const f4v lo = {a[0], a[1], a[2], a[3]}, hi = {a[4], a[5], a[6], a[7]};
+    __builtin_nontemporal_store(lo, reinterpret_cast<f4v*>(dst));
+    __builtin_nontemporal_store(hi, reinterpret_cast<f4v*>(dst) + 1);
+}
+
 // ------------------------------------------------------------------------------------------------ forward
 // out[row][b] = sum over the row's edges of w * state[source][b] (float32 sums); split rows write partial sums
-template <typename S>
+template <typename S, int PB>
 __global__ __launch_bounds__(WG) void k_fwd16(Plan p, const int2* __restrict__ cw, const unsigned short* __restrict__ src,
                                               int src_rows, float* __restrict__ out, int B, float* __restrict__ part,
                                               int T, int RB) {
@@ -70,8 +100,8 @@ __global__ __launch_bounds__(WG) void k_fwd16(Plan p, const int2* __restrict__ c
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
     const bool wok = load_wave(p, w, wv);
-    const int2* q = cw + wv.x + lane;
-    int2 nxt = (wok && wv.y > 0) ? q[0] : make_int2(NO_ROW, 0);
+    const PairLoad<PB> q(cw, wv.x, lane);
+    int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;
     const bool live = load_segment(p, w * 8 + (grp & 7), sg) && wok;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -80,12 +110,12 @@ __global__ __launch_bounds__(WG) void k_fwd16(Plan p, const int2* __restrict__ c
     for (int j = 0, left = wok ? wv.y : 0; left > 0; ++j, left -= 8) {
         int c[8];
         float wt[8];
-        stage8(slots[grp], sub, nxt, c, wt);
+        stage_pairs<PB>(slots, grp, sub, nxt, false, nullptr, src_rows, c, wt);
         u32x4 raw[8];
 #pragma unroll
         for (int s = 0; s < 8; ++s) raw[s] = s < left ? gather16(rs, c[s], sub) : u32x4{0u, 0u, 0u, 0u};
         __builtin_amdgcn_sched_barrier(0);
-        if (left > 8) nxt = q[64 * (j + 1)];
+        if (left > 8) nxt = q.step(j + 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
@@ -101,13 +131,13 @@ __global__ __launch_bounds__(WG) void k_fwd16(Plan p, const int2* __restrict__ c
         return;
     }
     const int b0 = tile * TW16 + sub * 8;
-    if (b0 < B) store8(out + (size_t)sg.x * B + b0, acc);
+    if (b0 < B) store8_stream(out + (size_t)sg.x * B + b0, acc);
 }
 
 // ------------------------------------------------------------------------------------------------ backward
 // Over the transposed plan (rows = sources j): gh[j][b] = scale * sum_e w_e gz[col_e][b], and per (plan position,
 // tile) the partial sum over the tile's samples of gz[col_e][b] * h[j][b] (the weight gradient before the scale).
-template <typename S>
+template <typename S, int PB>
 __global__ __launch_bounds__(WG) void k_bwd16(Plan p, const int2* __restrict__ cw, const unsigned short* __restrict__ gz,
                                               int gz_rows, const unsigned short* __restrict__ hs,
                                               float* __restrict__ gh, int B, float* __restrict__ gwpart, long long gw_ld,
@@ -120,8 +150,8 @@ __global__ __launch_bounds__(WG) void k_bwd16(Plan p, const int2* __restrict__ c
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
     const bool wok = load_wave(p, w, wv);
-    const int2* q = cw + wv.x + lane;
-    int2 nxt = (wok && wv.y > 0) ? q[0] : make_int2(NO_ROW, 0);
+    const PairLoad<PB> q(cw, wv.x, lane);
+    int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;
     const bool live = load_segment(p, w * 8 + (grp & 7), sg) && wok;
     float hj[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -133,31 +163,36 @@ __global__ __launch_bounds__(WG) void k_bwd16(Plan p, const int2* __restrict__ c
         (void*)(gz + (size_t)tile * gz_rows * TW16), (short)0, gz_rows * 128, 0x00020000);
     float* gwp = gwpart ? gwpart + (size_t)tile * gw_ld + wv.x + lane : nullptr;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int j = 0, left = wok ? wv.y : 0; left > 0; ++j, left -= 8) {
+    float pend = 0.f;                           // (a step's partial is stored after the next step's gathers: k_bwd)
+    int j = 0;
+    for (int left = wok ? wv.y : 0; left > 0; ++j, left -= 8) {
         int c[8];
         float wt[8];
-        stage8(slots[grp], sub, nxt, c, wt);
+        stage_pairs<PB>(slots, grp, sub, nxt, false, nullptr, gz_rows, c, wt);
         u32x4 raw[8];
 #pragma unroll
         for (int s = 0; s < 8; ++s) raw[s] = s < left ? gather16(rs, c[s], sub) : u32x4{0u, 0u, 0u, 0u};
         __builtin_amdgcn_sched_barrier(0);
-        if (left > 8) nxt = q[64 * (j + 1)];
+        if (left > 8) nxt = q.step(j + 1);
+        if (gwp && j > 0) __builtin_nontemporal_store(pend, gwp + 64 * (j - 1));
         __builtin_amdgcn_sched_barrier(0);
         float d[8];
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            float f[8];
-            unpack8<S>(raw[s], f);
             float dp = 0.f;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                acc[k] = fmaf(wt[s], f[k], acc[k]);
-                dp = fmaf(hj[k], f[k], dp);
+            for (int k = 0; k < 4; ++k) {
+                const unsigned g = raw[s][k];
+                acc[2 * k] = Bits16<S>::fma_lo(g, wt[s], acc[2 * k]);
+                dp = Bits16<S>::fma_lo(g, hj[2 * k], dp);
+                acc[2 * k + 1] = Bits16<S>::fma_hi(g, wt[s], acc[2 * k + 1]);
+                dp = Bits16<S>::fma_hi(g, hj[2 * k + 1], dp);
             }
             d[s] = dp;
         }
-        if (gwp) gwp[64 * j] = rs8(d, sub);
+        if (gwp) pend = rs8(d, sub);
     }
+    if (gwp && j > 0) __builtin_nontemporal_store(pend, gwp + 64 * (j - 1));
     if (!live) return;
     if (sg.y >= 0) {
         store8(part + ((size_t)tile * p.nslot + sg.y) * TW16 + sub * 8, acc);
@@ -168,7 +203,7 @@ __global__ __launch_bounds__(WG) void k_bwd16(Plan p, const int2* __restrict__ c
     const float sc = scale ? *scale : 1.f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) acc[k] *= sc;
-    store8(gh + (size_t)sg.x * B + b0, acc);
+    store8_stream(gh + (size_t)sg.x * B + b0, acc);
 }
 
 // split rows: their partial sums in segment order, times *mul (if given), into the row-major output
@@ -184,11 +219,20 @@ __global__ __launch_bounds__(WG) void k_comb16(Plan p, const float* __restrict__
     const int b0 = tile * TW16 + sub * 8;
     if (b0 >= B) return;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int k = 0; k < s.z; ++k) {
-        const float* src = part + ((size_t)tile * p.nslot + s.y + k) * TW16 + sub * 8;
-        const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
-        acc[0] += a.x; acc[1] += a.y; acc[2] += a.z; acc[3] += a.w;
-        acc[4] += b.x; acc[5] += b.y; acc[6] += b.z; acc[7] += b.w;
+    for (int k = 0; k < s.z; k += 8) {              // 8 loads in flight (past the end: the last slot, not added)
+        float4 a[8], b[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const float* src = part + ((size_t)tile * p.nslot + s.y + min(k + u, s.z - 1)) * TW16 + sub * 8;
+            a[u] = *reinterpret_cast<const float4*>(src);
+            b[u] = *reinterpret_cast<const float4*>(src + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (k + u < s.z) {
+                acc[0] += a[u].x; acc[1] += a[u].y; acc[2] += a[u].z; acc[3] += a[u].w;
+                acc[4] += b[u].x; acc[5] += b[u].y; acc[6] += b[u].z; acc[7] += b[u].w;
+            }
     }
     if (mul) {
         const float m = *mul;
@@ -247,7 +291,7 @@ void fh_absmax(const float* x, long long n, float* out, void* stream) {
     hipStream_t st = (hipStream_t)stream;
     FG_CHECK(launch_fill(out, 1e-30f, 1, st), );
     if (n == 0) return;
-    const long long nb = std::min<long long>(1024, (n + WG - 1) / WG);
+    const long long nb = std::min<long long>(2048, (n + WG - 1) / WG);
     k_absmax<<<(unsigned)nb, WG, 0, st>>>(x, n, (unsigned*)out);
     FG_CHECK(hipGetLastError(), );
 }
@@ -263,12 +307,16 @@ void fh_spmm_h(const int* wave, int nwave, const int* seg, int nseg, const int* 
     }
     hipStream_t st = (hipStream_t)stream;
     const int T = (B + TW16 - 1) / TW16;
-    FG_CHECK(launch_pack(pcol, pidx, w, (int2*)cw, npos, st), );
-    Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_rows, nslot, npos};
+    Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_rows, nslot, npos,
+           pair_width(n_src, npos, nwave)};
+    FG_CHECK(launch_pack(pcol, pidx, w, (int2*)cw, npos, st, p.pb), );
     if (nwave > 0) {
         const int RB = (nwave + WG / 64 - 1) / (WG / 64);
-        k_fwd16<F16><<<(unsigned)tile_blocks(RB, T), WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)hs, n_src,
-                                                                  out, B, scratch, T, RB);
+        const unsigned grid = (unsigned)tile_blocks(RB, T);
+        if (p.pb == 6)
+            k_fwd16<F16, 6><<<grid, WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)hs, n_src, out, B, scratch, T, RB);
+        else
+            k_fwd16<F16, 8><<<grid, WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)hs, n_src, out, B, scratch, T, RB);
         FG_CHECK(hipGetLastError(), );
     }
     if (nsplit > 0) {
@@ -289,13 +337,19 @@ void fh_spmm_bwd_h(const int* wave, int nwave, const int* seg, int nseg, const i
     }
     hipStream_t st = (hipStream_t)stream;
     const int T = (B + TW16 - 1) / TW16;
-    FG_CHECK(launch_pack(pcol, pidx, w, (int2*)cw, npos, st), );
-    Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_src, nslot, npos};
+    Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_src, nslot, npos,
+           pair_width(n_rows, npos, nwave)};
+    FG_CHECK(launch_pack(pcol, pidx, w, (int2*)cw, npos, st, p.pb), );
     if (nwave > 0) {
         const int RB = (nwave + WG / 64 - 1) / (WG / 64);
-        k_bwd16<F16><<<(unsigned)tile_blocks(RB, T), WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)gzs, n_rows,
-                                                                  (const unsigned short*)hs, gh, B, gw ? gwpart : nullptr,
-                                                                  npos, scale, scratch, T, RB);
+        const unsigned grid = (unsigned)tile_blocks(RB, T);
+        float* part = gw ? gwpart : nullptr;
+        if (p.pb == 6)
+            k_bwd16<F16, 6><<<grid, WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)gzs, n_rows,
+                                                 (const unsigned short*)hs, gh, B, part, npos, scale, scratch, T, RB);
+        else
+            k_bwd16<F16, 8><<<grid, WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)gzs, n_rows,
+                                                 (const unsigned short*)hs, gh, B, part, npos, scale, scratch, T, RB);
         FG_CHECK(hipGetLastError(), );
     }
     if (nsplit > 0) {

@@ -57,11 +57,12 @@ bool spmm_args_ok(const int* wave, int nwave, const int* seg, int nseg, const in
 void spmm_run(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
               const int* pcol, const int* pidx, long long npos, const float* w, const float* h, float* out, int n_rows,
               int n_src, int B, int2* cw, float* partials, hipStream_t st, bool h_tiled = false) {
-    FG_CHECK(launch_pack(pcol, pidx, w, cw, npos, st), );
     FwdEpi e;
     e.z = out;
     e.lz = plain(B);
-    Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_rows, nslot, npos};
+    Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_rows, nslot, npos,
+           h_tiled ? pair_width(n_src, npos, nwave) : 8};
+    FG_CHECK(launch_pack(pcol, pidx, w, cw, npos, st, p.pb), );
     FG_CHECK(launch_fwd(p, cw, h, h_tiled ? tiled(n_src) : plain(B), n_src, e, partials, tiled(nslot), B / TW, st), );
 }
 
@@ -81,12 +82,13 @@ void spmm_bwd_run(const int* wave, int nwave, const int* seg, int nseg, const in
                   float* gh, float* gw, int n_rows, int n_src, int B, int2* cw, float* gwpart, float* scratch,
                   hipStream_t st, bool gz_tiled) {
     const int T = B / TW;
-    FG_CHECK(launch_pack(pcol, pidx, w, cw, npos, st), );
     BwdEpi e;
     e.mode = 0;
     e.gh_out = gh;
     e.lgh = plain(B);
-    Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_src, nslot, npos};
+    Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_src, nslot, npos,
+           gz_tiled ? pair_width(n_rows, npos, nwave) : 8};
+    FG_CHECK(launch_pack(pcol, pidx, w, cw, npos, st, p.pb), );
     FG_CHECK(launch_bwd(p, cw, gz, gz_tiled ? tiled(n_rows) : plain(B), n_rows, h, plain(B), gw ? gwpart : nullptr,
                         npos, e, scratch, tiled(nslot), T, st), );
     if (gw) FG_CHECK(launch_reduce(gwpart, npos, npos, T, pidx, nullptr, gw, st), );

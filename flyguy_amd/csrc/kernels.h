@@ -113,6 +113,11 @@ struct BwdEpi {
 // cw[p] = (pcol[p], w[pidx[p]]) for the npos positions of a plan; pidx[p] < 0: (NO_ROW, 0)
 hipError_t launch_pack(const int* pcol, const int* pidx, const float* w, int2* cw, long long npos, hipStream_t st,
                        int pb = 8);   // pb 6 (Plan::pb): npos a multiple of 64
+// The pair storage of a tiled product whose pairs are packed on each call (the fh_* products; the caller's 8 bytes per
+// position hold either form), by the rule of the core's plans (pair_storage in core.hip)
+inline int pair_width(int gathered_rows, long long npos, int nwave) {
+    return gathered_rows <= PAIR6_MAX_ROWS && npos % 64 == 0 && npos / 64 >= 3LL * nwave ? 6 : 8;
+}
 // The tables a pass derives from one set of weights, a job each (k_derive).  A job's weights are given by their offset
 // in the set (floats); npos of a pair job is a multiple of 64.
 struct DeriveJob {

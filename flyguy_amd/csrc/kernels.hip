@@ -609,7 +609,7 @@ template <int MODE>
 __device__ __forceinline__ void bwd_finish(const BwdEpi& e, int j, int tile, int sub, float4 gh, const BwdIn& in,
                                            float2* keep = nullptr, int gcol = -1) {
     if constexpr (MODE == 0) {
-        *at4w(e.gh_out, e.lgh, tile, j, sub) = gh;
+        st_stream(at4w(e.gh_out, e.lgh, tile, j, sub), gh);
         return;
     }
     float4 gzv;

@@ -45,10 +45,30 @@ def _key(t: torch.Tensor | None):
     return None if t is None else (t.data_ptr(), t.numel(), t.device, t._version)
 
 
-def _plan(rowptr: torch.Tensor, col: torch.Tensor, idx: torch.Tensor | None, n_edges: int):
-    """The device plan of a product: its row plan, and per plan position the source row (col[edge]) and the weight
-    index (idx[edge], or the edge itself)."""
-    key = (_key(rowptr), _key(col), _key(idx))
+def _striped(p: dict) -> dict:
+    """A row plan whose longest wave is at least four times its middle one, with its waves dealt out so that each
+    workgroup of four takes one from each quarter (the rule and order of the library's own forwards, core.hip:striped);
+    other plans as they are.  Positions stay where they are: a wave's record names them."""
+    wave, seg = p["wave"], p["seg"]
+    n = len(wave)
+    if n == 0 or wave[0, 1] < 4 * max(int(wave[n // 2, 1]), 8):
+        return p
+    blocks = -(-n // 4)
+    order = (np.arange(blocks)[:, None] + blocks * np.arange(4)).reshape(-1)         # wave of place 4 block + i
+    there = order < n
+    out = np.zeros((4 * blocks, 2), np.int32)                                        # (a place past the plan: no steps)
+    out[there] = wave[order[there]]
+    groups = np.full((8 * n, 4), -1, np.int32)                                       # (a group without a segment)
+    groups[:len(seg)] = seg
+    segs = np.full((4 * blocks, 8, 4), -1, np.int32)
+    segs[there] = groups.reshape(n, 8, 4)[order[there]]
+    return dict(p, wave=out, seg=segs.reshape(-1, 4))
+
+
+def _plan(rowptr: torch.Tensor, col: torch.Tensor, idx: torch.Tensor | None, n_edges: int, forward: bool = False):
+    """The device plan of a product: its row plan (a forward's striped, _striped), and per plan position the source row
+    (col[edge]) and the weight index (idx[edge], or the edge itself)."""
+    key = (_key(rowptr), _key(col), _key(idx), forward)
     hit = _plans.get(key)
     if hit is not None and hit[0] is rowptr and hit[1] is col and hit[2] is idx:
         _plans.move_to_end(key)
@@ -57,6 +77,8 @@ def _plan(rowptr: torch.Tensor, col: torch.Tensor, idx: torch.Tensor | None, n_e
     if rp[0] != 0 or rp[-1] != n_edges or (len(rp) > 1 and (rp[1:] < rp[:-1]).any()):
         raise ValueError("HopHip: row pointer does not describe the connection arrays it came with")
     p = plan_rows(rp)
+    if forward:
+        p = _striped(p)
     pos = p["pos"].astype(np.int64)
     used = pos >= 0
     c = col.detach().cpu().numpy()
@@ -108,7 +130,7 @@ class HopHip(torch.autograd.Function):
         if w.numel() != E or col.dtype != torch.int32 or crow.dtype != torch.int64:
             raise ValueError("HopHip: w / col / crow do not match (float32 w[E], int32 col[E], int64 crow)")
         _check_index(col, n_src, "source index")
-        d = _plan(crow, col, None, E)
+        d = _plan(crow, col, None, E, forward=True)
         out = torch.empty(n_rows, B, device=h.device)
         cw = torch.empty(max(d["npos"], 1), 2, dtype=torch.int32, device=h.device)
         if half:
