@@ -48,6 +48,12 @@ _SIGS = {
     "fh_spmm_tiled": (None, [vp, ci, vp, ci, vp, ci, ci, vp, vp, cll, vp, vp, vp, ci, ci, ci, vp, vp, vp]),
     "fh_spmm_bwd_tiled": (None, [vp, ci, vp, ci, vp, ci, ci, vp, vp, cll, vp, vp, vp, vp, vp, ci, ci, ci, vp, vp, vp,
                                  vp]),
+    "fh_layer": (None, [vp, ci, vp, ci, vp, ci, ci, vp, vp, cll, vp, vp, vp, vp, ci, vp, ci, ci, ci, vp, vp, vp]),
+    "fh_layer_bwd": (None, [vp, ci, vp, ci, vp, ci, ci, vp, vp, cll, vp, vp, vp, vp, vp, ci, ci, ci, ci, vp, vp, vp,
+                            vp]),
+    "fh_redrive_bwd": (None, [vp, vp, ci, ci, ci, vp, vp]),
+    "fh_fire_tiled": (None, [vp, vp, vp, ci, ci, vp, vp]),
+    "fh_fire_bwd_tiled": (None, [vp, vp, vp, vp, ci, ci, vp, vp, vp, vp]),
     "fh_absmax": (None, [vp, cll, vp, vp]),
     "fh_spmm_h": (None, [vp, ci, vp, ci, vp, ci, ci, vp, vp, cll, vp, vp, vp, ci, ci, ci, vp, vp, vp]),
     "fh_spmm_bwd_h": (None, [vp, ci, vp, ci, vp, ci, ci, vp, vp, cll, vp, vp, vp, vp, vp, vp, ci, ci, ci, vp, vp, vp,

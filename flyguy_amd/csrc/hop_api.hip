@@ -52,14 +52,29 @@ bool spmm_args_ok(const int* wave, int nwave, const int* seg, int nseg, const in
              (nsplit > 0 && !split));
 }
 
+// the rest of a layer's input, with a tiled output: a bias per row, and the drive (tiled, n_s rows) that the plan's re-drive
+// fields name rows of
+struct LayerIn {
+    const float* bias;
+    const float* drive;
+    int n_s;
+};
+
 // pack the pairs into cw, then the product through the plan (split rows' partial sums in `partials`); h row-major
 // [n_src][B], or tiled [B/32][n_src][32] (h_tiled)
 void spmm_run(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
               const int* pcol, const int* pidx, long long npos, const float* w, const float* h, float* out, int n_rows,
-              int n_src, int B, int2* cw, float* partials, hipStream_t st, bool h_tiled = false) {
+              int n_src, int B, int2* cw, float* partials, hipStream_t st, bool h_tiled = false,
+              const LayerIn* layer = nullptr) {
     FwdEpi e;
     e.z = out;
     e.lz = plain(B);
+    if (layer) {
+        e.lz = tiled(n_rows);
+        e.after = layer->bias;
+        e.drive = layer->drive;
+        e.ldrive = tiled(layer->n_s);
+    }
     Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_rows, nslot, npos,
            h_tiled ? pair_width(n_src, npos, nwave) : 8};
     FG_CHECK(launch_pack(pcol, pidx, w, cw, npos, st, p.pb), );
@@ -80,18 +95,19 @@ bool spmm_bwd_args_ok(const int* wave, int nwave, const int* seg, int nseg, cons
 void spmm_bwd_run(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
                   const int* pcol, const int* pidx, long long npos, const float* w, const float* gz, const float* h,
                   float* gh, float* gw, int n_rows, int n_src, int B, int2* cw, float* gwpart, float* scratch,
-                  hipStream_t st, bool gz_tiled) {
+                  hipStream_t st, bool gz_tiled, bool all_tiled = false, bool pair = false) {
     const int T = B / TW;
     BwdEpi e;
     e.mode = 0;
     e.gh_out = gh;
-    e.lgh = plain(B);
+    e.lgh = all_tiled ? tiled(n_src) : plain(B);
     Plan p{(const int2*)wave, nwave, (const int4*)seg, nseg, (const int4*)split, nsplit, n_src, nslot, npos,
            gz_tiled ? pair_width(n_rows, npos, nwave) : 8};
     FG_CHECK(launch_pack(pcol, pidx, w, cw, npos, st, p.pb), );
-    FG_CHECK(launch_bwd(p, cw, gz, gz_tiled ? tiled(n_rows) : plain(B), n_rows, h, plain(B), gw ? gwpart : nullptr,
-                        npos, e, scratch, tiled(nslot), T, st), );
-    if (gw) FG_CHECK(launch_reduce(gwpart, npos, npos, T, pidx, nullptr, gw, st), );
+    FG_CHECK(launch_bwd(p, cw, gz, gz_tiled ? tiled(n_rows) : plain(B), n_rows, h,
+                        all_tiled ? tiled(n_src) : plain(B), gw ? gwpart : nullptr, npos, e, scratch, tiled(nslot), T, st,
+                        pair), );
+    if (gw) FG_CHECK(launch_reduce(gwpart, npos, npos, pair ? (T + 1) / 2 : T, pidx, nullptr, gw, st), );
 }
 
 // one 8-lane group per (tile, row): a row's 128-byte line of the tile, row-major -> tiled
@@ -118,13 +134,14 @@ __device__ __forceinline__ float fire1(float g, float z, float t) {
     return a > 0.f ? a : (a != a ? a : 0.f);
 }
 
+// TILED: z and h are [B/32][rows][32] (q: the rows), else [rows][B] (q: the float4 per row).
 // I: the index type (32-bit unless the states hold 2^31 float4 or more: its division is the cheaper one)
-template <class I>
+template <class I, bool TILED>
 __global__ __launch_bounds__(WG) void k_fire(const float4* __restrict__ z, const float* __restrict__ g,
                                              const float* __restrict__ t, I q, I n, float4* __restrict__ h) {
-    const I i = (I)blockIdx.x * WG + threadIdx.x;                           // q float4 per row
+    const I i = (I)blockIdx.x * WG + threadIdx.x;
     if (i >= n) return;
-    const int r = (int)(i / q);
+    const int r = (int)(TILED ? (i >> 3) % q : i / q);
     const float gr = g[r], tr = t[r];
     const float4 v = z[i];
     h[i] = make_float4(fire1(gr, v.x, tr), fire1(gr, v.y, tr), fire1(gr, v.z, tr), fire1(gr, v.w, tr));
@@ -132,7 +149,9 @@ __global__ __launch_bounds__(WG) void k_fire(const float4* __restrict__ z, const
 
 // Its backward, one workgroup per row: where g z - t is not <= 0 (positive, or NaN: PyTorch's relu passes the
 // gradient of a NaN on) gz = gh g, elsewhere 0, and the row's gradients of g and t, gg = sum gh z and gt = -sum gh
-// over those samples (each product rounded, as PyTorch forms them; the sums in this kernel's order)
+// over those samples (each product rounded, as PyTorch forms them; the sums in this kernel's order, the same for both
+// layouts).  TILED: gh, z and gz are [B/32][rows][32], else [rows][B]; q float4 per row.
+template <bool TILED>
 __global__ __launch_bounds__(WG) void k_fire_bwd(const float4* __restrict__ gh, const float4* __restrict__ z,
                                                  const float* __restrict__ g, const float* __restrict__ t, int q,
                                                  float4* __restrict__ gz, float* __restrict__ gg,
@@ -142,7 +161,7 @@ __global__ __launch_bounds__(WG) void k_fire_bwd(const float4* __restrict__ gh, 
     const float gr = g[r], tr = t[r];
     float sz = 0.f, s1 = 0.f;
     for (int k = threadIdx.x; k < q; k += WG) {
-        const size_t i = (size_t)r * q + k;
+        const size_t i = TILED ? ((size_t)(k >> 3) * gridDim.x + r) * LPR + (k & 7) : (size_t)r * q + k;
         const float4 v = z[i], d = gh[i];
         const float zv[4] = {v.x, v.y, v.z, v.w}, dv[4] = {d.x, d.y, d.z, d.w};
         float o[4];
@@ -174,6 +193,31 @@ __global__ __launch_bounds__(WG) void k_fire_bwd(const float4* __restrict__ gh, 
         gg[r] = a;
         gt[r] = -b;
     }
+}
+
+// out [B/32][n_s][32]: row j of a tile is row inv[j] of gz [B/32][rows][32], or zero where inv[j] is none (the gradient
+// that re-driven rows send to the drive): one pass, where a clearing, a gather and a scatter move every line three times
+__global__ __launch_bounds__(WG) void k_redrive_bwd(const float* __restrict__ gz, int rows, const int* __restrict__ inv,
+                                                    int n_s, float* __restrict__ out, long long n) {
+    const long long i = (long long)blockIdx.x * WG + threadIdx.x;
+    if (i >= n) return;
+    const int sub = (int)(i & 7), j = (int)((i >> 3) % n_s), tile = (int)((i >> 3) / n_s), r = inv[j];
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if ((unsigned)r < (unsigned)rows) v = reinterpret_cast<const float4*>(gz)[((size_t)tile * rows + r) * LPR + sub];
+    reinterpret_cast<float4*>(out)[i] = v;
+}
+
+template <bool TILED>
+void fire_run(const float* z, const float* g, const float* t, int rows, int B, float* h, hipStream_t st) {
+    const long long n = (long long)rows * (B / 4), q = TILED ? rows : B / 4;
+    if (n == 0) return;
+    const unsigned blocks = (unsigned)((n + WG - 1) / WG);
+    if (n < (1LL << 31))
+        k_fire<unsigned, TILED><<<blocks, WG, 0, st>>>((const float4*)z, g, t, (unsigned)q, (unsigned)n, (float4*)h);
+    else
+        k_fire<unsigned long long, TILED><<<blocks, WG, 0, st>>>((const float4*)z, g, t, (unsigned long long)q,
+                                                                 (unsigned long long)n, (float4*)h);
+    FG_CHECK(hipGetLastError(), );
 }
 
 }  // namespace
@@ -276,16 +320,7 @@ void fh_fire(const float* z, const float* g, const float* t, int rows, int B, fl
         set_error("fh_fire: bad argument");
         return;
     }
-    const long long n = (long long)rows * (B / 4);
-    if (n == 0) return;
-    const unsigned blocks = (unsigned)((n + WG - 1) / WG);
-    if (n < (1LL << 31))
-        k_fire<unsigned><<<blocks, WG, 0, (hipStream_t)stream>>>((const float4*)z, g, t, (unsigned)(B / 4), (unsigned)n,
-                                                                 (float4*)h);
-    else
-        k_fire<unsigned long long><<<blocks, WG, 0, (hipStream_t)stream>>>(
-            (const float4*)z, g, t, (unsigned long long)(B / 4), (unsigned long long)n, (float4*)h);
-    FG_CHECK(hipGetLastError(), );
+    fire_run<false>(z, g, t, rows, B, h, (hipStream_t)stream);
 }
 
 void fh_fire_bwd(const float* gh, const float* z, const float* g, const float* t, int rows, int B, float* gz, float* gg,
@@ -296,8 +331,70 @@ void fh_fire_bwd(const float* gh, const float* z, const float* g, const float* t
         return;
     }
     if (rows == 0) return;
-    k_fire_bwd<<<(unsigned)rows, WG, 0, (hipStream_t)stream>>>((const float4*)gh, (const float4*)z, g, t, B / 4,
+    k_fire_bwd<false><<<(unsigned)rows, WG, 0, (hipStream_t)stream>>>((const float4*)gh, (const float4*)z, g, t, B / 4,
                                                                 (float4*)gz, gg, gt);
+    FG_CHECK(hipGetLastError(), );
+}
+
+void fh_layer(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
+              const int* pcol, const int* pidx, long long npos, const float* w, const float* ht, const float* bias,
+              const float* drive, int n_s, float* out, int n_rows, int n_src, int B, void* cw, float* scratch,
+              void* stream) {
+    clear_error();
+    if (!spmm_args_ok(wave, nwave, seg, nseg, split, nsplit, nslot, pcol, pidx, npos, w, ht, out, n_rows, n_src, B) ||
+        (nwave > 0 && !cw) || (nsplit > 0 && !scratch) || (drive && n_s <= 0)) {
+        set_error("fh_layer: bad argument");
+        return;
+    }
+    const LayerIn in{bias, drive, n_s};
+    spmm_run(wave, nwave, seg, nseg, split, nsplit, nslot, pcol, pidx, npos, w, ht, out, n_rows, n_src, B, (int2*)cw,
+             scratch, (hipStream_t)stream, true, &in);
+}
+
+void fh_layer_bwd(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
+                  const int* pcol, const int* pidx, long long npos, const float* w, const float* gzt, const float* ht,
+                  float* ght, float* gw, int n_rows, int n_src, int B, int pair, void* cw, float* gwpart, float* scratch,
+                  void* stream) {
+    clear_error();
+    if (!spmm_bwd_args_ok(wave, nwave, seg, nseg, split, nsplit, nslot, pcol, pidx, npos, w, gzt, ht, ght, gw, n_rows,
+                          n_src, B, cw, gwpart, scratch)) {
+        set_error("fh_layer_bwd: bad argument");
+        return;
+    }
+    spmm_bwd_run(wave, nwave, seg, nseg, split, nsplit, nslot, pcol, pidx, npos, w, gzt, ht, ght, gw, n_rows, n_src, B,
+                 (int2*)cw, gwpart, scratch, (hipStream_t)stream, true, true, pair != 0);
+}
+
+void fh_redrive_bwd(const float* gzt, const int* inv, int rows, int n_s, int B, float* out, void* stream) {
+    clear_error();
+    if (!gzt || !inv || !out || rows <= 0 || n_s <= 0 || B <= 0 || B % TW) {
+        set_error("fh_redrive_bwd: bad argument");
+        return;
+    }
+    const long long n = (long long)n_s * (B / 4);
+    k_redrive_bwd<<<(unsigned)((n + WG - 1) / WG), WG, 0, (hipStream_t)stream>>>(gzt, rows, inv, n_s, out, n);
+    FG_CHECK(hipGetLastError(), );
+}
+
+void fh_fire_tiled(const float* z, const float* g, const float* t, int rows, int B, float* h, void* stream) {
+    clear_error();
+    if (!z || !g || !t || !h || rows < 0 || B <= 0 || B % TW) {
+        set_error("fh_fire_tiled: bad argument");
+        return;
+    }
+    fire_run<true>(z, g, t, rows, B, h, (hipStream_t)stream);
+}
+
+void fh_fire_bwd_tiled(const float* gh, const float* z, const float* g, const float* t, int rows, int B, float* gz,
+                       float* gg, float* gt, void* stream) {
+    clear_error();
+    if (!gh || !z || !g || !t || !gz || !gg || !gt || rows < 0 || B <= 0 || B % TW) {
+        set_error("fh_fire_bwd_tiled: bad argument");
+        return;
+    }
+    if (rows == 0) return;
+    k_fire_bwd<true><<<(unsigned)rows, WG, 0, (hipStream_t)stream>>>((const float4*)gh, (const float4*)z, g, t, B / 4,
+                                                                      (float4*)gz, gg, gt);
     FG_CHECK(hipGetLastError(), );
 }
 

@@ -64,6 +64,7 @@ struct FwdEpi {
                                       // a bias, whole rows take it from sinfo (the records' fourth field)
     const float* drive = nullptr;     // the sensory layer's drive, for re-drive rows (nullptr: none in this layer)
     Lay ldrive{};
+    const float* after = nullptr;     // per row: added to the row's sum (where bias starts it)
     float* z = nullptr;               // the pre-activation: stored for the sensory layer (the drive) and raw products
     Lay lz{};
     float* h = nullptr;
@@ -185,9 +186,9 @@ __host__ __device__ inline int fires_bytes_ld(int rows) { return (rows + 31) / 3
 constexpr int FIRES_LDS_WORDS = 8192;
 // bytes [T][fires_bytes_ld(rows)] (FwdEpi::fires) -> bitmaps [T][fires_ld(rows)]
 hipError_t launch_fires_pack(const unsigned char* bytes, int rows, unsigned* bits, int T, hipStream_t st);
-// gwpart: the per-position weight-gradient partials, gw_ld apart, one row per tile; with pair (a tiled layer backward,
-// modes 1 and 2, whose hsrc must be epi.h: the layer's own output) one row per pair of tiles (tiles 2p and 2p + 1
-// summed), ceil(T / 2) rows, and so are the rows' gain and threshold partials (epi.ggain_part, epi.gsum_part)
+// gwpart: the per-position weight-gradient partials, gw_ld apart, one row per tile; with pair (tiled; in modes 1 and 2
+// hsrc must be epi.h: the layer's own output) one row per pair of tiles (tiles 2p and 2p + 1 summed), ceil(T / 2) rows,
+// and so are the rows' gain and threshold partials (epi.ggain_part, epi.gsum_part)
 hipError_t launch_bwd(const Plan& p, const int2* cw, const float* gz, Lay lg, int gz_rows, const float* hsrc, Lay lhs,
                       float* gwpart, long long gw_ld, const BwdEpi& epi, float* part, Lay lp, int T, hipStream_t st,
                       bool pair = false);

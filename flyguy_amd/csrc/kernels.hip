@@ -155,6 +155,7 @@ __device__ __forceinline__ void st_stream(float4* p, const float4& v) {
 // (the lanes of whole 8-lane groups call this together)
 __device__ __forceinline__ void fwd_finish(const FwdEpi& e, int t, int tile, int sub, float4 acc, const FwdIn& in) {
     if (e.drive) add4(in.dv, acc);              // (zero when the row has no re-drive)
+    if (e.after) add4(splat(e.after[t]), acc);
     if (e.z) st_stream(at4w(e.z, e.lz, tile, t, sub), acc);
     if (e.info) {
         const float g = in.g, sp = in.sp;
@@ -765,7 +766,8 @@ __global__ __launch_bounds__(WG) void k_bwd2(Plan p, const int2* __restrict__ cw
         hja = ld_stream(at4u(hs, lhs, ta, sg.x, sub));
         if (hasb) hjb = ld_stream(at4u(hs, lhs, tb, sg.x, sub));
     }
-    const bool quiet_a = epi.skip_silent && group_silent(hja), quiet_b = epi.skip_silent && group_silent(hjb);
+    const bool skip = MODE != 0 && epi.skip_silent;
+    const bool quiet_a = skip && group_silent(hja), quiet_b = skip && group_silent(hjb);
     const Slab<true> sa(gz + (size_t)ta * lg.tile, lg.row, gz_rows, sub);
     const Slab<true> sb(gz + (size_t)(hasb ? tb : ta) * lg.tile, lg.row, gz_rows, sub);
     float* gwp = gwpart ? gwpart + (size_t)pr * gw_ld + wv.x + lane : nullptr;
@@ -814,7 +816,7 @@ __global__ __launch_bounds__(WG) void k_bwd2(Plan p, const int2* __restrict__ cw
     float2 ka, kb = make_float2(0.f, 0.f);
     bwd_finish<MODE>(epi, sg.x, ta, sub, acca, ina, &ka);
     if (hasb) bwd_finish<MODE>(epi, sg.x, tb, sub, accb, inb, &kb);
-    if (sub == 0) {                             // the row's gain and threshold partials, one per pair of tiles
+    if (MODE != 0 && sub == 0) {                             // the row's gain and threshold partials, one per pair of tiles
         const int col = w * 8 + (grp & 7);      // (the plan column of the row: its segment)
         epi.ggain_part[(size_t)pr * epi.gp_ld + col] = ka.x + kb.x;
         epi.gsum_part[(size_t)pr * epi.gp_ld + col] = ka.y + kb.y;
@@ -1502,7 +1504,7 @@ static void launch_bwd_kernel(const Plan& p, const int2* cw, const float* gz, La
                               Lay lhs, float* gwpart, long long gw_ld, const BwdEpi& epi, float* part, Lay lp, int T,
                               bool pair, hipStream_t st) {
     const int RB = (p.nwave + WG / 64 - 1) / (WG / 64);
-    if constexpr (TILED && MODE != 0) {
+    if constexpr (TILED) {
         if (pair) {                             // two tiles per workgroup
             k_bwd2<MODE, PB><<<(unsigned)tile_blocks(RB, (T + 1) / 2), WG, 0, st>>>(p, cw, gz, lg, gz_rows, hsrc, lhs,
                                                                                      gwpart, gw_ld, epi, part, lp, T, RB);
@@ -1551,8 +1553,9 @@ hipError_t launch_bwd(const Plan& p, const int2* cw, const float* gz, Lay lg, in
     const bool tiled_ = lg.row == TW;
     switch (epi.mode) {
         case 0:
+            if (pair && (lhs.row != TW || !tiled_)) return hipErrorInvalidValue;
             return tiled_ ? launch_bwd_as<true, 0>(p, cw, gz, lg, gz_rows, hsrc, lhs, gwpart, gw_ld, epi, part, lp, T,
-                                                   false, st)
+                                                   pair, st)
                           : launch_bwd_as<false, 0>(p, cw, gz, lg, gz_rows, hsrc, lhs, gwpart, gw_ld, epi, part, lp, T,
                                                     false, st);
         case 1:

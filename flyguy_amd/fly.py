@@ -285,6 +285,31 @@ class FlyActor(nn.Module):
         top = h.index_select(axis, self.dn_rows)
         return self.out(top.t() if by_neuron else top)
 
+    def _walk_tiled(self, obs: torch.Tensor) -> torch.Tensor:
+        """_walk on the library's float32 kernels with the states [B/32, rows, 32] throughout (HopHip's layer form): a
+        layer's product, bias and re-driven rows are one pass, and no state is copied from one layout to the other."""
+        from .fly_hip import FireHip, HopHip
+        B = obs.shape[0]
+        thr = nn.functional.softplus(self.theta)
+        layers = self._layers()
+
+        def product(layer, w, h, bias, drive):
+            p = layer.prod
+            given = drive is not None and len(layer.redriven) > 0
+            return HopHip.apply(w, h, p.crow, p.ci, p.tcrow, p.tci, p.tperm, False, bias, drive if given else None,
+                                layer.redriven if given else None, layer.drive_rows if given else None)
+
+        def fire(z, nid):
+            return FireHip.apply(z, self.gain.index_select(0, nid), thr.index_select(0, nid))
+
+        x = obs.reshape(B // 32, 32, obs.shape[1]).transpose(1, 2).contiguous()
+        drive = product(layers[0], self.in_w, x, self.in_b, None)
+        h = fire(drive, layers[0].nid)
+        for layer in layers[1:]:
+            h = fire(product(layer, self.w.index_select(0, layer.edges), h, None, drive), layer.nid)
+        top = h.index_select(1, self.dn_rows)
+        return self.out(top.transpose(1, 2).reshape(B, -1))
+
     # ---- CPU play
     def _host_decider(self) -> "_HostDecider | None":
         """The CPU decision library loaded with the current weights (rebuilt when a weight changed), or None when it
@@ -340,6 +365,8 @@ class FlyActor(nn.Module):
         if self.kernel != "torch" and obs.is_cuda and obs.shape[0] % 32 == 0:      # (at any batch size)
             from .fly_hip import FireHip, HopHip
             half = self.kernel == "cuda16"
+            if not half and self.w.dtype == torch.float32 and obs.shape[0]:
+                return self._walk_tiled(obs)
 
             def on_library(k, layer, w, h):
                 p = layer.prod

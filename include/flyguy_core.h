@@ -215,6 +215,28 @@ void fh_spmm_bwd_tiled(const int* wave, int nwave, const int* seg, int nseg, con
                        float* gh, float* gw, int n_rows, int n_src, int B, void* cw, float* gwpart, float* scratch,
                        void* stream);
 
+/* ---- a layer's input with every state tiled ([B/32][rows][32]), for FlyActor's GPU path; no counterpart in the
+ * reference ---- */
+
+/* out (tiled, n_rows) = A ht, each row's sum plus bias[row] (null: none) and plus row d of drive (tiled, n_s rows; null:
+ * none) where the row's re-drive field in the plan is d >= 0 (third int of a segment, fourth of a split row; -1 none,
+ * below n_s).  Other arguments as fh_spmm_tiled. */
+void fh_layer(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
+              const int* pcol, const int* pidx, long long npos, const float* w, const float* ht, const float* bias,
+              const float* drive, int n_s, float* out, int n_rows, int n_src, int B, void* cw, float* scratch,
+              void* stream);
+
+/* fh_spmm_bwd with gzt, ht and ght tiled.  pair: two tiles per workgroup, which halves the weight-gradient partials
+ * (gwpart: npos * ceil(B/64) floats then) and pays where few rows of gz take most of the gathers. */
+void fh_layer_bwd(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
+                  const int* pcol, const int* pidx, long long npos, const float* w, const float* gzt, const float* ht,
+                  float* ght, float* gw, int n_rows, int n_src, int B, int pair, void* cw, float* gwpart, float* scratch,
+                  void* stream);
+
+/* out (tiled, n_s rows): row j is row inv[j] of gzt (tiled, `rows` of them), zeros where inv[j] < 0: the drive's
+ * gradient from one layer's re-driven rows. */
+void fh_redrive_bwd(const float* gzt, const int* inv, int rows, int n_s, int B, float* out, void* stream);
+
 /* ---- the neuron activation of FlyActor's GPU path, h = relu(g z - t) per row, for the PyTorch elementwise steps of
  * fly.py:296-304 (fire).  No counterpart in the library of the reference: its GPU actor path (fly.py:170-185) forms
  * it from three PyTorch operations, each a pass over the states.  z, h: [rows][B] row-major float32, B % 4 == 0;
@@ -227,6 +249,11 @@ void fh_fire(const float* z, const float* g, const float* t, int rows, int B, fl
  * samples. */
 void fh_fire_bwd(const float* gh, const float* z, const float* g, const float* t, int rows, int B, float* gz, float* gg,
                  float* gt, void* stream);
+
+/* The same over tiled states ([B/32][rows][32], B % 32 == 0): the same values, and the same sums in the same order. */
+void fh_fire_tiled(const float* z, const float* g, const float* t, int rows, int B, float* h, void* stream);
+void fh_fire_bwd_tiled(const float* gh, const float* z, const float* g, const float* t, int rows, int B, float* gz,
+                       float* gg, float* gt, void* stream);
 
 /* ---- 16-bit states (the reference's half path, fly_cuda.py:34-56, 93-115): products read states and gradients as
  * IEEE binary16 and accumulate in float32.  A 16-bit state tensor is tiled: [ceil(B/64)][rows][64] halves, samples
