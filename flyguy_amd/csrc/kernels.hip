@@ -480,7 +480,8 @@ __global__ __launch_bounds__(WG) void k_touch(TouchJob j) {
     asm volatile("" ::"v"(acc));                                   // (the loads are kept; nothing is stored)
 }
 
-// split rows: partial sums in segment order, then the same finish
+// split rows: partial sums in segment order, then the same finish.  From COMBINE_FEW rows and tiles up one 8-lane group
+// per row and tile, which keeps the chip's loads busy; below, k_fwd_combine_few.
 // acc += the n partial sums of (slots y .., tile), in slot order, 8 loads in flight
 __device__ __forceinline__ void add_parts(const float* __restrict__ part, Lay lp, int tile, int y, int n, int sub,
                                           float4& acc) {
@@ -507,6 +508,35 @@ __global__ __launch_bounds__(WG) void k_fwd_combine(Plan p, const float* __restr
     const FwdIn in = fwd_inputs(epi, epi.info, s.x, s.w, tile, sub);
     add_parts(part, lp, tile, s.y, s.z, sub, acc);
     fwd_finish(epi, s.x, tile, sub, acc, in);
+}
+
+// The same for few split rows and tiles, where the launch is over when the row of most partial sums is (80 to 113 on the
+// networks measured, 8 loads in flight and the last up to 7 one by one): one wave per row and tile, whose 8 groups load
+// 64 slots at once and hand them over in LDS; every group then adds them in slot order, k_fwd_combine's sums bit for bit.
+// One tile of the benchmark network, hop 1 / 2 / 3: 5.1 / 5.4 / 8.4 -> 3.9 / 4.5 / 3.9 us.
+__global__ __launch_bounds__(64) void k_fwd_combine_few(Plan p, const float* __restrict__ part, Lay lp, FwdEpi epi) {
+    __shared__ float4 slot[64][LPR];
+    const int tile = blockIdx.y, grp = threadIdx.x >> 3, sub = threadIdx.x & 7;
+    int4 s;
+    if (!load_split(p, blockIdx.x, s)) return;
+    const int n = __builtin_amdgcn_readfirstlane(s.z), d = __builtin_amdgcn_readfirstlane(s.w);
+    float4 acc = epi.bias ? splat(epi.bias[s.x]) : splat(0.f);
+    FwdIn in{};
+    for (int k = 0; k < n; k += 64) {
+        const int m = min(n - k, 64);
+        float4 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (8 * u < m) v[u] = ld_stream(at4(part, lp, tile, s.y + k + min(8 * u + grp, m - 1), sub));
+        if (k == 0) in = fwd_inputs(epi, epi.info, s.x, d, tile, sub);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (8 * u < m) slot[8 * u + grp][sub] = v[u];
+        __builtin_amdgcn_wave_barrier();
+        for (int i = 0; i < m; ++i) add4(slot[i][sub], acc);
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (grp == 0) fwd_finish(epi, s.x, tile, sub, acc, in);
 }
 
 // One workgroup per tile: the tile's firing bytes -> its bitmap (bits, then the count of silent rows in the header)
@@ -1388,6 +1418,16 @@ hipError_t launch_derive(const DeriveJob* jobs, const int* first, int njobs, lon
     return hipGetLastError();
 }
 
+// At 13 tiles (5.3 / 6.4 / 9.4 thousand rows and tiles) k_fwd_combine takes 5.8 / 5.0 / 7.7 us and k_fwd_combine_few 5.4 /
+// 5.3 / 7.4; at 16 tiles (6.5 / 7.8 / 11.6) 5.8 / 5.3 / 7.6 and 5.9 / 5.6 / 8.2.
+constexpr long long COMBINE_FEW = 6000;
+static void combine_fwd(const Plan& p, const float* part, Lay lp, const FwdEpi& epi, int T, hipStream_t st) {
+    if ((long long)p.nsplit * T <= COMBINE_FEW)
+        k_fwd_combine_few<<<dim3((unsigned)p.nsplit, (unsigned)T), 64, 0, st>>>(p, part, lp, epi);
+    else
+        k_fwd_combine<<<blocks((long long)p.nsplit * T * LPR), WG, 0, st>>>(p, part, lp, epi, T);
+}
+
 hipError_t launch_fwd(const Plan& p, const int2* cw, const float* src, Lay ls, int src_rows, const FwdEpi& epi,
                       float* part, Lay lp, int T, hipStream_t st, const unsigned* src_fires) {
     // 6-byte pairs name rows by 16 bits: only a tiled slab of at most PAIR6_MAX_ROWS rows reads 0xFFFF as past its end
@@ -1420,7 +1460,7 @@ hipError_t launch_fwd(const Plan& p, const int2* cw, const float* src, Lay ls, i
         if (e != hipSuccess) return e;
     }
     if (p.nsplit > 0) {
-        k_fwd_combine<<<blocks((long long)p.nsplit * T * LPR), WG, 0, st>>>(p, part, lp, epi, T);
+        combine_fwd(p, part, lp, epi, T, st);
         return hipGetLastError();
     }
     return hipSuccess;
@@ -1448,7 +1488,7 @@ hipError_t launch_fwd_lds(const Plan& p, const int2* cw, const float* src, int s
         if (e != hipSuccess) return e;
     }
     if (p.nsplit > 0) {
-        k_fwd_combine<<<blocks((long long)p.nsplit * T * LPR), WG, 0, st>>>(p, part, lp, epi, T);
+        combine_fwd(p, part, lp, epi, T, st);
         return hipGetLastError();
     }
     return hipSuccess;

@@ -92,3 +92,48 @@ def test_few_tiles(gpu_lib, uneven, monkeypatch, tiles):
         got.append([core.forward(obs)] + [core.state(k, 0, n, B) for k, n in enumerate(s["sizes"])])
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_rows_of_many_segments(gpu_lib, bias):
+    """Rows of 1 to 130 partial sums (64 of them are loaded at once for few tiles, 8 for many): bit for bit the same for
+    one tile and for a batch of 1,000, and within float32 sums of the float64 product."""
+    segments = [1, 2, 7, 8, 9, 63, 64, 65, 128, 130]
+    rng = np.random.default_rng(3)
+    n_src, B = 4000, 32000
+    deg = [16 * k - 3 for k in segments]
+    crow = np.concatenate([[0], np.cumsum(deg)])
+    col = np.concatenate([np.sort(rng.choice(n_src, d, replace=False)) for d in deg])
+    order = np.argsort(col, kind="stable")
+    tcrow = np.concatenate([[0], np.cumsum(np.bincount(col, minlength=n_src))])
+    row = np.repeat(np.arange(len(deg)), deg)
+    put = lambda a, t: torch.as_tensor(np.ascontiguousarray(a, dtype=t)).cuda()      # noqa: E731
+    index = (put(crow, np.int64), put(col, np.int32), put(tcrow, np.int64), put(row[order], np.int32),
+             put(order, np.int64))
+    g = torch.Generator(device="cuda").manual_seed(1)
+    w = torch.randn(len(col), device="cuda", generator=g)
+    h = torch.randn(B // 32, n_src, 32, device="cuda", generator=g)
+    b = torch.randn(len(deg), device="cuda", generator=g) if bias else None
+    layer = (False, b, None, None, None)
+    many = HopHip.apply(w, h, *index, *layer)
+    for tile in (0, 1, B // 32 - 1):
+        assert torch.equal(HopHip.apply(w, h[tile:tile + 1].contiguous(), *index, *layer)[0], many[tile])
+    dense = torch.zeros(len(deg), n_src, device="cuda", dtype=torch.float64)
+    dense[put(row, np.int64), put(col, np.int64)] = w.double()
+    want = dense @ h[0].double() + (b.double()[:, None] if bias else 0)
+    # a sum of n terms in float32 is off by at most n 2^-24 of the sum of their magnitudes
+    bound = (put(deg, np.float64)[:, None] + 2) * 2.0 ** -24 * (dense.abs() @ h[0].double().abs() + 4)
+    assert ((many[0].double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("n_dn", [500, 513, 1332, 1700])
+def test_read_out_of_any_batch(gpu_lib, n_dn, bf16):
+    """The read-out keeps more of a wave's 8-row groups in flight up to 1,024 samples (1, 2, 3 or 4 groups at these
+    sizes): logits bit for bit those of a larger batch."""
+    s, params = synth_3hop(sizes=(600, 900, 800, n_dn), edges=(9_000, 8_000, 12_000), redrive=(60, 20, 2))
+    obs = np.random.default_rng(n_dn).standard_normal((1088, s["obs_dim"])).astype(np.float32)
+    core = Core(s, params, 1088, int(bf16))
+    want = core.forward(obs)
+    for n in (64, 1024):
+        assert np.array_equal(core.forward(obs[:n]), want[:n]), n
