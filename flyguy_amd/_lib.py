@@ -23,6 +23,8 @@ _SIGS = {
     "fc_forward": (None, [vp, vp, ci, vp, ci]),
     "fc_zero_grad": (None, [vp]),
     "fc_backward": (None, [vp, vp, ci]),
+    "fc_forward_n": (None, [vp, vp, ci, vp, ci]),
+    "fc_backward_n": (None, [vp, vp, ci]),
     "fc_grad_norm": (cf, [vp]),
     "fc_step": (cf, [vp, cf, cf, cf, cf, cf]),
     "fc_adam_t": (cll, [vp, cll]),

@@ -183,7 +183,8 @@ bool check_batch(const Core* c, int B);
 bool prof_collect(Core& c);
 // forward of a batch through the weight set `set` (SET_P or SET_EMA); obs [B][obs_dim] row-major on the device;
 // logits [B][n_act]
-bool forward(Core& c, const float* obs, int B, float* logits, int set);
+// (n: obs and logits hold the first n of the B samples only, the others repeat the last one's; -1: all)
+bool forward(Core& c, const float* obs, int B, float* logits, int set, int n = -1);
 // backward of the last forward (through SET_P) from dlogits [B][n_act]: gradients ADDED to the SET_G arrays
 // fresh: the gradient starts from zero and this backward is the only one adding to it (a teaching step), so the first
 // sum into each entry is stored instead of added (no read of the entry)

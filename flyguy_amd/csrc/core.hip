@@ -10,6 +10,7 @@
 //           not kept: the backward needs it only where h > 0, and there it is (h + softplus(theta)) / gain);
 //   partial sums: split rows, per-edge weight gradients [T or T/2][E_k], per-row gain / threshold gradients [T][rows],
 //                 plug gradients [T][n_s] / [T][E_in], read-out gradients [chunks][n_act * n_dn].
+#include <climits>
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -792,7 +793,7 @@ static bool plan_tables(Core& c) {
     return c.djobs && c.dfirst;
 }
 
-static bool forward16(Core& c, const float* obs, int B, float* logits, int set);
+static bool forward16(Core& c, const float* obs, int B, float* logits, int set, int n);
 static bool backward16(Core& c, const float* dlogits, int B, bool fresh);
 
 // Workgroups per tile of the plug staged in LDS (launch_fwd_lds; launch_plug_bwd_lds for its gradients), or 0 for
@@ -819,11 +820,12 @@ static bool fwd_skips(const Core& c, const HopD& d, int T, bool bf16) {
     return (long long)d.E * T >= FIRES_MIN_LINES && (bf16 || !fwd_deep(d.fp.view(), T));
 }
 
-bool forward(Core& c, const float* obs, int B, float* logits, int set) {
-    if (c.prec) return forward16(c, obs, B, logits, set);
+bool forward(Core& c, const float* obs, int B, float* logits, int set, int n) {
+    if (n < 0) n = B;
+    if (c.prec) return forward16(c, obs, B, logits, set, n);
     const int T = B / TW;
     hipStream_t st = c.st;
-    { Timed t(c, ST_OBS); FG_CHECK(launch_obs_in(obs, c.x, c.obs_dim, B, st), false); }
+    { Timed t(c, ST_OBS); FG_CHECK(launch_obs_in(obs, c.x, c.obs_dim, B, n, st), false); }
     if (!derive(c, set, true, false)) return false;
     const bool old_tables = c.tables_old;       // (the caches have moved on since they were made: see the plug below)
     c.tables_old = true;
@@ -882,7 +884,7 @@ bool forward(Core& c, const float* obs, int B, float* logits, int set) {
     {
         Timed t(c, ST_LOGITS);
         FG_CHECK(launch_logits_mfma(hp, false, c.sizes[c.hops], c.dn, c.n_dn, c.arr(set, 6), c.n_act, c.owT, c.lpart, logits,
-                                    B, st), false);
+                                    B, n, st), false);
     }
     c.B = B;
     return true;
@@ -989,10 +991,10 @@ bool backward(Core& c, const float* dlogits, int B, bool fresh) {
 typedef unsigned short u16;
 static u16* s16(float* p) { return reinterpret_cast<u16*>(p); }
 
-static bool forward16(Core& c, const float* obs, int B, float* logits, int set) {
+static bool forward16(Core& c, const float* obs, int B, float* logits, int set, int n) {
     const int T = B / TW16;
     hipStream_t st = c.st;
-    { Timed t(c, ST_OBS); FG_CHECK(launch_obs_in16(obs, s16(c.x), c.obs_dim, B, st), false); }
+    { Timed t(c, ST_OBS); FG_CHECK(launch_obs_in16(obs, s16(c.x), c.obs_dim, B, n, st), false); }
     if (!derive(c, set, true, false)) return false;
     auto skips = [&](int layer) { return layer < c.hops && fwd_skips(c, c.hop[(size_t)layer], T, true); };   // (as forward)
     auto bytes = [&](int layer) { return skips(layer) ? c.fire_bytes[(size_t)layer] : nullptr; };
@@ -1035,7 +1037,7 @@ static bool forward16(Core& c, const float* obs, int B, float* logits, int set) 
     {
         Timed t(c, ST_LOGITS);
         FG_CHECK(launch_logits_mfma(hp, true, c.sizes[c.hops], c.dn, c.n_dn, c.arr(set, 6), c.n_act, c.owT, c.lpart, logits,
-                                    B, st), false);
+                                    B, n, st), false);
     }
     c.B = B;
     return true;
@@ -1262,6 +1264,34 @@ void fc_forward(void* h, const float* obs, int B, float* logits, int ema) {
     if (!check_batch(c, B)) return;
     if (!obs || !logits) { set_error("fc_forward: null pointer"); return; }
     forward(*c, obs, B, logits, ema ? SET_EMA : SET_P);
+}
+
+// n samples as a batch of whole tiles (0 and an error where the handle holds no such batch)
+static int ragged_batch(const Core* c, int n) {
+    const int q = c && c->prec ? TW16 : TW;
+    const int B = n > 0 && n <= INT_MAX - q ? (n + q - 1) / q * q : n;
+    return check_batch(c, B) ? B : 0;
+}
+
+void fc_forward_n(void* h, const float* obs, int n, float* logits, int ema) {
+    Core* c = (Core*)h;
+    const int B = ragged_batch(c, n);
+    if (!B) return;
+    if (!obs || !logits) { set_error("fc_forward_n: null pointer"); return; }
+    forward(*c, obs, B, logits, ema ? SET_EMA : SET_P, n);
+}
+
+void fc_backward_n(void* h, const float* dlogits, int n) {
+    Core* c = (Core*)h;
+    const int B = ragged_batch(c, n);
+    if (!B) return;
+    if (!dlogits) { set_error("fc_backward_n: null pointer"); return; }
+    if (B != c->B) { set_error("fc_backward_n: batch differs from the last forward's"); return; }
+    if (n < B) {
+        FG_CHECK(launch_pad(dlogits, (long long)n * c->n_act, c->dl, (long long)B * c->n_act, c->st), );
+        dlogits = c->dl;
+    }
+    backward(*c, dlogits, B);
 }
 
 void fc_zero_grad(void* h) {

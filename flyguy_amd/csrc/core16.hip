@@ -600,12 +600,13 @@ __global__ __launch_bounds__(WG) void k_cbwd16_combine(Plan p, const float* __re
 
 // ------------------------------------------------------------------------------------------------ x, read-out
 // obs [B][obs_dim] float32 -> x [T][obs_dim][64] bfloat16; one workgroup per (tile, 64 features)
-__global__ __launch_bounds__(WG) void k_obs_in16(const float* __restrict__ obs, bf16_t* __restrict__ x, int obs_dim) {
+__global__ __launch_bounds__(WG) void k_obs_in16(const float* __restrict__ obs, bf16_t* __restrict__ x, int obs_dim,
+                                                 int n) {
     __shared__ float s[TW16][65];
     const int tile = blockIdx.y, f0 = blockIdx.x * 64;
     for (int i = threadIdx.x; i < TW16 * 64; i += WG) {
         const int c = i / 64, f = i % 64;
-        s[c][f] = (f0 + f < obs_dim) ? obs[(size_t)(tile * TW16 + c) * obs_dim + f0 + f] : 0.f;
+        s[c][f] = (f0 + f < obs_dim) ? obs[(size_t)min(tile * TW16 + c, n - 1) * obs_dim + f0 + f] : 0.f;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < TW16 * 64; i += WG) {
@@ -644,8 +645,8 @@ __global__ void k_export16(const bf16_t* __restrict__ src, int rows, float* __re
 // ------------------------------------------------------------------------------------------------ launchers
 static inline unsigned nblocks(long long n, int per = WG) { return (unsigned)((n + per - 1) / per); }
 
-hipError_t launch_obs_in16(const float* obs, unsigned short* x, int obs_dim, int B, hipStream_t st) {
-    k_obs_in16<<<dim3((unsigned)((obs_dim + 63) / 64), (unsigned)(B / TW16)), WG, 0, st>>>(obs, x, obs_dim);
+hipError_t launch_obs_in16(const float* obs, unsigned short* x, int obs_dim, int B, int n, hipStream_t st) {
+    k_obs_in16<<<dim3((unsigned)((obs_dim + 63) / 64), (unsigned)(B / TW16)), WG, 0, st>>>(obs, x, obs_dim, n);
     return hipGetLastError();
 }
 

@@ -211,7 +211,8 @@ constexpr int WLDS_COLD = 1 << 30;
 hipError_t launch_bwd_lds(const Plan& p, const int2* wlds, const int2* cw, const float* gz, int gz_rows,
                           const int* hot_rows, int hot, const float* hsrc, Lay lhs, float* gwpart, long long gw_ld,
                           const BwdEpi& epi, float* part, Lay lp, int T, int S, hipStream_t st);
-hipError_t launch_obs_in(const float* obs, float* x, int obs_dim, int B, hipStream_t st);
+// obs [n][obs_dim] into the tiled x of B samples, the last row repeated from n on
+hipError_t launch_obs_in(const float* obs, float* x, int obs_dim, int B, int n, hipStream_t st);
 // the read-out on the matrix cores (readout.hip): owT, the weights transposed, n_dn x
 // readout_pad(n_act); hK float32 tiles of 32 or (bf16_states) bfloat16 tiles of 64
 int readout_pad(int n_act);
@@ -219,10 +220,10 @@ hipError_t launch_readout_bwd_w_mfma(const float* dl, const void* hK, bool bf16_
                                      int n_dn, int n_act, float* gow_part, float* gob_part, int B, hipStream_t st);
 hipError_t launch_readout_bwd_h_mfma(const float* dl, const float* owT, const int* dn_inv, int n_act, int rows,
                                      const BwdEpi& epi, int B, hipStream_t st);
-// lpart: RO_SPLIT x B x n_act floats of scratch (the sums over each split of the read-out rows)
+// logits: of the n first of the B samples.  lpart: RO_SPLIT x B x n_act floats of scratch (the sums over each split of the read-out rows)
 constexpr int RO_SPLIT = 8;
 hipError_t launch_logits_mfma(const void* hK, bool bf16_states, int rows, const int* dn, int n_dn, const float* ob,
-                              int n_act, const float* owT, float* lpart, float* logits, int B, hipStream_t st);
+                              int n_act, const float* owT, float* lpart, float* logits, int B, int n, hipStream_t st);
 // the read-out weights' gradient partials come per chunk of RO_CHUNK_S samples: readout_chunks(B) of them
 constexpr int RO_CHUNK_S = 128;
 int readout_chunks(int B);
@@ -282,7 +283,7 @@ struct BwdEpi16 {
     float* ginw_part = nullptr;
     long long gw_ld = 0;
 };
-hipError_t launch_obs_in16(const float* obs, unsigned short* x, int obs_dim, int B, hipStream_t st);
+hipError_t launch_obs_in16(const float* obs, unsigned short* x, int obs_dim, int B, int n, hipStream_t st);
 hipError_t launch_fwd16c(const Plan& p, const int2* cw, const unsigned short* src, int src_rows, const FwdEpi16& epi,
                          float* part, int T, hipStream_t st, const unsigned* src_fires = nullptr);
 // the same with each tile's source slab staged in LDS (launch_fwd_lds)
@@ -307,6 +308,8 @@ hipError_t launch_readout_bwd_h16_mfma(const float* dl, const float* owT, const 
 hipError_t launch_loss(const float* lg, const float* tl, float* dl, float* stats_part, float* stats, int n_act, int B,
                        float it, hipStream_t st, bool accumulate = false);
 hipError_t launch_fill(float* p, float v, long long n, hipStream_t st);
+// dst[0 .. total) = src[0 .. n), then zeros
+hipError_t launch_pad(const float* src, long long n, float* dst, long long total, hipStream_t st);
 // up to 7 arrays of floats copied in one launch (source and destination: memory of the current device, apart)
 struct CopyJobs {
     const float* src[7] = {};

@@ -1150,12 +1150,12 @@ __global__ __launch_bounds__(BWD_LDS_NW * 64) void k_bwd_lds(Plan p, const int2*
 
 // ------------------------------------------------------------------------------------------------ obs / logits
 // obs [B][obs_dim] (row-major, the caller's) -> x [T][obs_dim][32]; one workgroup per (tile, 64 features)
-__global__ __launch_bounds__(WG) void k_obs_in(const float* __restrict__ obs, float* __restrict__ x, int obs_dim) {
+__global__ __launch_bounds__(WG) void k_obs_in(const float* __restrict__ obs, float* __restrict__ x, int obs_dim, int n) {
     __shared__ float s[TW][65];
     const int tile = blockIdx.y, f0 = blockIdx.x * 64;
     for (int i = threadIdx.x; i < TW * 64; i += WG) {
         const int c = i / 64, f = i % 64;
-        s[c][f] = (f0 + f < obs_dim) ? obs[(size_t)(tile * TW + c) * obs_dim + f0 + f] : 0.f;
+        s[c][f] = (f0 + f < obs_dim) ? obs[(size_t)min(tile * TW + c, n - 1) * obs_dim + f0 + f] : 0.f;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < TW * 64; i += WG) {
@@ -1322,6 +1322,12 @@ __global__ __launch_bounds__(WG) void k_sum_pairs(const float* __restrict__ part
 __global__ void k_fill(float* __restrict__ p, float v, long long n) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
+}
+
+__global__ __launch_bounds__(WG) void k_pad(const float* __restrict__ src, long long n, float* __restrict__ dst,
+                                            long long total) {
+    const long long i = (long long)blockIdx.x * WG + threadIdx.x;
+    if (i < total) dst[i] = i < n ? src[i] : 0.f;
 }
 
 // Array k of the jobs by the blocks (., k), 16 bytes a thread and turn where both ends are aligned for it.  Seven copies
@@ -1669,9 +1675,9 @@ hipError_t launch_fires_pack(const unsigned char* bytes, int rows, unsigned* bit
     return hipGetLastError();
 }
 
-hipError_t launch_obs_in(const float* obs, float* x, int obs_dim, int B, hipStream_t st) {
+hipError_t launch_obs_in(const float* obs, float* x, int obs_dim, int B, int n, hipStream_t st) {
     dim3 grid((unsigned)((obs_dim + 63) / 64), (unsigned)(B / TW));
-    k_obs_in<<<grid, WG, 0, st>>>(obs, x, obs_dim);
+    k_obs_in<<<grid, WG, 0, st>>>(obs, x, obs_dim, n);
     return hipGetLastError();
 }
 
@@ -1714,6 +1720,11 @@ hipError_t launch_loss(const float* lg, const float* tl, float* dl, float* stats
 hipError_t launch_fill(float* p, float v, long long n, hipStream_t st) {
     if (n <= 0) return hipSuccess;
     k_fill<<<blocks(n), WG, 0, st>>>(p, v, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_pad(const float* src, long long n, float* dst, long long total, hipStream_t st) {
+    k_pad<<<blocks(total), WG, 0, st>>>(src, n, dst, total);
     return hipGetLastError();
 }
 

@@ -92,14 +92,15 @@ __global__ __launch_bounds__(64 * RO_WAVES) void k_logits_mfma(const void* __res
     }
 }
 
-// logits[b][a] = ob[a] + the RO_SPLIT partial sums of k_logits_mfma, added in split order
+// logits[b][a] = ob[a] + the RO_SPLIT partial sums of k_logits_mfma (ld apart), added in split order, for the n first
 __global__ __launch_bounds__(WG) void k_logits_sum(const float* __restrict__ lpart, const float* __restrict__ ob,
-                                                   int n_act, long long n, float* __restrict__ logits) {
+                                                   int n_act, long long n, long long ld,
+                                                   float* __restrict__ logits) {
     const long long i = (long long)blockIdx.x * WG + threadIdx.x;
     if (i >= n) return;
     float v = lpart[i];
 #pragma unroll
-    for (int s = 1; s < RO_SPLIT; ++s) v += lpart[(size_t)s * n + i];
+    for (int s = 1; s < RO_SPLIT; ++s) v += lpart[(size_t)s * ld + i];
     logits[i] = ob[i % n_act] + v;
 }
 
@@ -197,12 +198,12 @@ hipError_t launch_readout_bwd_w_mfma(const float* dl, const void* hK, bool bf16_
 }
 
 hipError_t launch_logits_mfma(const void* hK, bool bf16_states, int rows, const int* dn, int n_dn, const float* ob,
-                              int n_act, const float* owT, float* lpart, float* logits, int B, hipStream_t st) {
+                              int n_act, const float* owT, float* lpart, float* logits, int B, int n, hipStream_t st) {
     const int ma = readout_pad(n_act);
-    if (ma > 32 * RO_MAXB || B % 32 != 0) return hipErrorInvalidValue;
+    if (ma > 32 * RO_MAXB || B % 32 != 0 || n > B) return hipErrorInvalidValue;
     const size_t sm = (size_t)((n_dn + 3) & ~3) * sizeof(int) + (size_t)RO_WAVES * 32 * 33 * sizeof(float);
     if (sm > 64 * 1024) return hipErrorInvalidValue;
-    if (B == 0) return hipSuccess;
+    if (B == 0 || n <= 0) return hipSuccess;
     const dim3 grid((unsigned)(B / 32), RO_SPLIT);
     const unsigned threads = 64 * RO_WAVES;
 #define FG_LOGITS(H, N) k_logits_mfma<H, N><<<grid, threads, sm, st>>>(hK, rows, H ? TW16 : TW, dn, n_dn, owT, ma, n_act, lpart)
@@ -215,8 +216,8 @@ hipError_t launch_logits_mfma(const void* hK, bool bf16_states, int rows, const 
 #undef FG_LOGITS
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const long long nl = (long long)B * n_act;
-    k_logits_sum<<<(unsigned)((nl + WG - 1) / WG), WG, 0, st>>>(lpart, ob, n_act, nl, logits);
+    const long long nl = (long long)n * n_act;
+    k_logits_sum<<<(unsigned)((nl + WG - 1) / WG), WG, 0, st>>>(lpart, ob, n_act, nl, (long long)B * n_act, logits);
     return hipGetLastError();
 }
 

@@ -40,10 +40,6 @@ TILE = 32                      # the library's batch granule (samples per tile)
 WEIGHTS, AVERAGE, ADAM_M, ADAM_V, GRADIENT = 0, 1, 2, 3, 4
 
 
-def _tile_up(n: int) -> int:
-    return -(-n // TILE) * TILE
-
-
 def _pieces(n: int, cap: int) -> list[slice]:
     """A batch of n samples as consecutive slices of at most cap samples."""
     return [slice(i, min(i + cap, n)) for i in range(0, n, cap)]
@@ -63,6 +59,7 @@ class _Session:
             raise RuntimeError("fc_create_from_memory failed")
         self.handle = handle
         self.stream = None
+        self.obs_dim = int(s["obs_dim"])
         self.evaluations = 0               # forward passes run so far (the library holds the last one's states)
         dev = actor.gain.device
         self.wmap = torch.as_tensor(np.asarray(s["wmap"], np.int64), device=dev)
@@ -100,27 +97,23 @@ class _Session:
         call("fc_copy", self.handle, which, 1 if into_library else 0, ptrs)
 
     def evaluate(self, obs: torch.Tensor, n_act: int) -> torch.Tensor:
-        """Logits of one piece (at most max_batch samples), padded to the tile granule by repeating the last row."""
+        """Logits of one piece (at most max_batch samples; the library fills the last tile with its last row)."""
         n = obs.shape[0]
-        pad = _tile_up(n) - n
-        x = torch.cat([obs, obs[-1:].expand(pad, obs.shape[1])]) if pad else obs
-        x = x.contiguous()
-        logits = torch.empty(x.shape[0], n_act, device=x.device)
+        if obs.numel() < n * self.obs_dim or (obs.dim() != 2 and n % TILE):
+            raise ValueError("NativeFlyActor: observations must be [samples, obs_dim]")
+        x = obs.contiguous()
+        logits = torch.empty(n, n_act, device=x.device)
         self.on_current_stream(x.device)
-        call("fc_forward", self.handle, x.data_ptr(), x.shape[0], logits.data_ptr(), 0)
+        call("fc_forward_n", self.handle, x.data_ptr(), n, logits.data_ptr(), 0)
         self.evaluations += 1
-        return logits[:n]
+        return logits
 
     def backpropagate(self, grad: torch.Tensor) -> None:
-        """The logits' gradient of the last evaluated piece (zero rows pad it to the granule); adds to the gradient."""
-        n = grad.shape[0]
-        pad = _tile_up(n) - n
-        g = grad.float()
-        if pad:
-            g = torch.cat([g, g.new_zeros(pad, g.shape[1])])
-        g = g.contiguous()
+        """The logits' gradient of the last evaluated piece (no gradient from the rest of the last tile); adds to the
+        gradient."""
+        g = grad.float().contiguous()
         self.on_current_stream(g.device)
-        call("fc_backward", self.handle, g.data_ptr(), g.shape[0])
+        call("fc_backward_n", self.handle, g.data_ptr(), g.shape[0])
 
 
 class _LibraryLogits(torch.autograd.Function):

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from flyguy_amd._lib import call
 from flyguy_amd.fly_hip import HopHip
 from flyguy_amd.synth import scaled_3hop, synth_3hop
 from gpu_helpers import NAMES, Core, rel
@@ -137,3 +138,33 @@ def test_read_out_of_any_batch(gpu_lib, n_dn, bf16):
     want = core.forward(obs)
     for n in (64, 1024):
         assert np.array_equal(core.forward(obs[:n]), want[:n]), n
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 65, 96, 100])
+def test_any_number_of_samples(gpu_lib, net, n, bf16):
+    """fc_forward_n and fc_backward_n against whole tiles padded by the caller (the last row repeated, no gradient):
+    logits and gradients bit for bit, and nothing written past the n-th sample's logits."""
+    s, params = net
+    B = 128
+    rng = np.random.default_rng(n)
+    obs = rng.standard_normal((n, s["obs_dim"])).astype(np.float32)
+    dl = rng.standard_normal((n, s["n_act"])).astype(np.float32)
+    core = Core(s, params, B, int(bf16))
+    whole = -(-n // (64 if bf16 else 32)) * (64 if bf16 else 32)
+    core.zero_grad()
+    want = core.forward(np.concatenate([obs, np.repeat(obs[-1:], whole - n, 0)]))
+    core.backward(np.concatenate([dl, np.zeros((whole - n, s["n_act"]), np.float32)]))
+    grads = core.get(4)
+    core.zero_grad()
+    x, d = torch.as_tensor(obs).cuda(), torch.as_tensor(dl).cuda()
+    logits = torch.full((n + 1, s["n_act"]), 7.0, device="cuda")
+    call("fc_forward_n", core.h, x.data_ptr(), n, logits.data_ptr(), 0)
+    call("fc_backward_n", core.h, d.data_ptr(), n)
+    torch.cuda.synchronize()
+    assert np.array_equal(logits[:n].cpu().numpy(), want[:n]) and bool((logits[n] == 7).all())
+    for name, a, b in zip(NAMES, grads, core.get(4)):
+        assert np.array_equal(a, b), name
+    for bad in (0, -1, 129, 2**31 - 1):
+        with pytest.raises(RuntimeError):
+            call("fc_forward_n", core.h, x.data_ptr(), bad, logits.data_ptr(), 0)
