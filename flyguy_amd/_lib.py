@@ -60,6 +60,8 @@ _SIGS = {
     "fh_spmm_h": (None, [vp, ci, vp, ci, vp, ci, ci, vp, vp, cll, vp, vp, vp, ci, ci, ci, vp, vp, vp]),
     "fh_spmm_bwd_h": (None, [vp, ci, vp, ci, vp, ci, ci, vp, vp, cll, vp, vp, vp, vp, vp, vp, ci, ci, ci, vp, vp, vp,
                              vp]),
+    "fh_spmm_bwd_h_pair": (None, [vp, ci, vp, ci, vp, ci, ci, vp, vp, cll, vp, vp, vp, vp, vp, vp, ci, ci, ci, ci, vp, vp,
+                                  vp, vp]),
     # include/flyguy_train.h
     "ft_main": (ci, [ci, ctypes.POINTER(ctypes.c_char_p)]),
     "ft_draw": (ci, [ctypes.c_ulonglong, ctypes.POINTER(cll), ci, ci, ci, vp]),

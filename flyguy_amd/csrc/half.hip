@@ -7,6 +7,8 @@
 // kernels (kernels.hip); the epilogues write the caller's row-major float32 [rows][B] outputs.
 #include <algorithm>
 
+#include <type_traits>
+
 #include "../../include/flyguy_core.h"
 #include "half.h"
 
@@ -206,6 +208,96 @@ __global__ __launch_bounds__(WG) void k_bwd16(Plan p, const int2* __restrict__ c
     store8_stream(gh + (size_t)sg.x * B + b0, acc);
 }
 
+// k_bwd16 with two tiles per workgroup (as the core's k_cbwd16x2, and chosen by its rule): a step's pairs are loaded once
+// for both, and one partial sum per pair of tiles is stored and read back.  The state gradient's sums are k_bwd16's, term
+// for term; a position's partial adds the second tile's products to the first's.
+template <typename S, int PB>
+__global__ __launch_bounds__(WG) void k_bwd16x2(Plan p, const int2* __restrict__ cw, const unsigned short* __restrict__ gz,
+                                                int gz_rows, const unsigned short* __restrict__ hs,
+                                                float* __restrict__ gh, int B, float* __restrict__ gwpart,
+                                                long long gw_ld, const float* __restrict__ scale,
+                                                float* __restrict__ part, int T, int RB) {
+    __shared__ __align__(16) int2 slots[WG / LPR][LPR];
+    int rb;
+    const int pr = tile_of(blockIdx.x, RB, (T + 1) / 2, rb);
+    if (rb >= RB) return;
+    const int ta = 2 * pr, tb = 2 * pr + 1;
+    const bool hasb = tb < T;
+    const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
+    int2 wv;
+    const bool wok = load_wave(p, w, wv);
+    const PairLoad<PB> q(cw, wv.x, lane);
+    int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
+    int4 sg;
+    const bool live = load_segment(p, w * 8 + (grp & 7), sg) && wok;
+    u32x4 ha{0u, 0u, 0u, 0u}, hb{0u, 0u, 0u, 0u};
+    if (live) {
+        ha = *reinterpret_cast<const u32x4*>(hs + ((size_t)ta * p.rows + sg.x) * TW16 + sub * 8);
+        if (hasb) hb = *reinterpret_cast<const u32x4*>(hs + ((size_t)tb * p.rows + sg.x) * TW16 + sub * 8);
+    }
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(gz + (size_t)ta * gz_rows * TW16), (short)0, gz_rows * 128, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb_ = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(gz + (size_t)(hasb ? tb : ta) * gz_rows * TW16), (short)0, gz_rows * 128, 0x00020000);
+    float* gwp = gwpart ? gwpart + (size_t)pr * gw_ld + wv.x + lane : nullptr;
+    float aa[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, ab[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float hja[8], hjb[8];
+    unpack8<S>(ha, hja);
+    unpack8<S>(hb, hjb);
+    float pend = 0.f;
+    int j = 0;
+    for (int left = wok ? wv.y : 0; left > 0; ++j, left -= 8) {
+        int c[8];
+        float wt[8];
+        stage_pairs<PB>(slots, grp, sub, nxt, false, nullptr, gz_rows, c, wt);
+        u32x4 va[8], vb[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) va[s] = s < left ? gather16(ra, c[s], sub) : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int s = 0; s < 8; ++s) vb[s] = hasb && s < left ? gather16(rb_, c[s], sub) : u32x4{0u, 0u, 0u, 0u};
+        __builtin_amdgcn_sched_barrier(0);
+        if (left > 8) nxt = q.step(j + 1);
+        if (gwp && j > 0) __builtin_nontemporal_store(pend, gwp + 64 * (j - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        float d[8];
+        auto add = [&](const u32x4 (&v)[8], const float (&hj)[8], float (&acc)[8], auto first) __attribute__((always_inline)) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                float dp = first.value ? 0.f : d[s];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const unsigned g = v[s][k];
+                    acc[2 * k] = Bits16<S>::fma_lo(g, wt[s], acc[2 * k]);
+                    dp = Bits16<S>::fma_lo(g, hj[2 * k], dp);
+                    acc[2 * k + 1] = Bits16<S>::fma_hi(g, wt[s], acc[2 * k + 1]);
+                    dp = Bits16<S>::fma_hi(g, hj[2 * k + 1], dp);
+                }
+                d[s] = dp;
+            }
+        };
+        add(va, hja, aa, std::true_type{});
+        add(vb, hjb, ab, std::false_type{});
+        if (gwp) pend = rs8(d, sub);
+    }
+    if (gwp && j > 0) __builtin_nontemporal_store(pend, gwp + 64 * (j - 1));
+    if (!live) return;
+    if (sg.y >= 0) {
+        store8(part + ((size_t)ta * p.nslot + sg.y) * TW16 + sub * 8, aa);
+        if (hasb) store8(part + ((size_t)tb * p.nslot + sg.y) * TW16 + sub * 8, ab);
+        return;
+    }
+    const float sc = scale ? *scale : 1.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        aa[k] *= sc;
+        ab[k] *= sc;
+    }
+    const int ba = ta * TW16 + sub * 8, bb = tb * TW16 + sub * 8;
+    if (ba < B) store8_stream(gh + (size_t)sg.x * B + ba, aa);
+    if (bb < B) store8_stream(gh + (size_t)sg.x * B + bb, ab);
+}
+
 // split rows: their partial sums in segment order, times *mul (if given), into the row-major output
 __global__ __launch_bounds__(WG) void k_comb16(Plan p, const float* __restrict__ part, float* __restrict__ out, int B,
                                                const float* __restrict__ mul, int T) {
@@ -329,6 +421,14 @@ void fh_spmm_bwd_h(const int* wave, int nwave, const int* seg, int nseg, const i
                    const int* pcol, const int* pidx, long long npos, const float* w, const void* gzs, const void* hs,
                    const float* scale, float* gh, float* gw, int n_rows, int n_src, int B, void* cw, float* gwpart,
                    float* scratch, void* stream) {
+    fh_spmm_bwd_h_pair(wave, nwave, seg, nseg, split, nsplit, nslot, pcol, pidx, npos, w, gzs, hs, scale, gh, gw, n_rows,
+                       n_src, B, 0, cw, gwpart, scratch, stream);
+}
+
+void fh_spmm_bwd_h_pair(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
+                        const int* pcol, const int* pidx, long long npos, const float* w, const void* gzs,
+                        const void* hs, const float* scale, float* gh, float* gw, int n_rows, int n_src, int B, int pair,
+                        void* cw, float* gwpart, float* scratch, void* stream) {
     clear_error();
     if (B <= 0 || B % TW || n_rows <= 0 || n_src <= 0 || !w || !gzs || !hs || !scale || !gh || (gw && !gwpart) ||
         !plan_args_ok(nwave, nseg, nsplit, nslot, npos, wave, seg, split, pcol, pidx, cw, scratch)) {
@@ -342,14 +442,16 @@ void fh_spmm_bwd_h(const int* wave, int nwave, const int* seg, int nseg, const i
     FG_CHECK(launch_pack(pcol, pidx, w, (int2*)cw, npos, st, p.pb), );
     if (nwave > 0) {
         const int RB = (nwave + WG / 64 - 1) / (WG / 64);
-        const unsigned grid = (unsigned)tile_blocks(RB, T);
+        const unsigned grid = (unsigned)tile_blocks(RB, pair ? (T + 1) / 2 : T);
         float* part = gw ? gwpart : nullptr;
-        if (p.pb == 6)
-            k_bwd16<F16, 6><<<grid, WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)gzs, n_rows,
-                                                 (const unsigned short*)hs, gh, B, part, npos, scale, scratch, T, RB);
-        else
-            k_bwd16<F16, 8><<<grid, WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)gzs, n_rows,
-                                                 (const unsigned short*)hs, gh, B, part, npos, scale, scratch, T, RB);
+#define FG_BWD16(K, P) K<F16, P><<<grid, WG, 0, st>>>(p, (const int2*)cw, (const unsigned short*)gzs, n_rows, \
+                                                      (const unsigned short*)hs, gh, B, part, npos, scale, scratch, T, RB)
+        if (p.pb == 6) {
+            if (pair) FG_BWD16(k_bwd16x2, 6); else FG_BWD16(k_bwd16, 6);
+        } else {
+            if (pair) FG_BWD16(k_bwd16x2, 8); else FG_BWD16(k_bwd16, 8);
+        }
+#undef FG_BWD16
         FG_CHECK(hipGetLastError(), );
     }
     if (nsplit > 0) {
@@ -357,7 +459,7 @@ void fh_spmm_bwd_h(const int* wave, int nwave, const int* seg, int nseg, const i
         FG_CHECK(hipGetLastError(), );
     }
     if (gw && npos > 0) {
-        k_reduce_mul<<<nblocks(npos), WG, 0, st>>>(gwpart, npos, npos, T, pidx, scale, gw);
+        k_reduce_mul<<<nblocks(npos), WG, 0, st>>>(gwpart, npos, npos, pair ? (T + 1) / 2 : T, pidx, scale, gw);
         FG_CHECK(hipGetLastError(), );
     }
 }

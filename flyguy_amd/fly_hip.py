@@ -186,7 +186,7 @@ class HopHip(torch.autograd.Function):
                  cw.data_ptr(), scratch.data_ptr(), _stream(h))
             ctx.hs = None
         ctx.save_for_backward(w, h, tcrow, tcol, tperm)
-        ctx.n_rows, ctx.half = n_rows, half
+        ctx.n_rows, ctx.half, ctx.pair = n_rows, half, d["pair"]
         return out
 
     @staticmethod
@@ -212,10 +212,12 @@ class HopHip(torch.autograd.Function):
             call("fh_absmax", gz.data_ptr(), gz.numel(), scale.data_ptr(), _stream(gz))
             gzs = torch.empty(max(t64 * ctx.n_rows * 64, 1), dtype=torch.float16, device=h.device)
             call("fh_to_half", gz.data_ptr(), ctx.n_rows, B, scale.data_ptr(), gzs.data_ptr(), _stream(gz))
-            gwpart = torch.empty(max(d["npos"] * t64, 1), device=h.device) if gw is not None else None
+            pair = ctx.pair and t64 > 1      # two tiles per workgroup where the core's backward takes two (pair_tiles)
+            gwpart = torch.empty(max(d["npos"] * (-(-t64 // 2) if pair else t64), 1),
+                                 device=h.device) if gw is not None else None
             scratch = torch.empty(max(d["nslot"] * t64 * 64, 1), device=h.device)
-            call("fh_spmm_bwd_h", *_args(d), w.data_ptr(), gzs.data_ptr(), ctx.hs.data_ptr(), scale.data_ptr(),
-                 gh.data_ptr(), gw.data_ptr() if gw is not None else None, ctx.n_rows, n_src, B, cw.data_ptr(),
+            call("fh_spmm_bwd_h_pair", *_args(d), w.data_ptr(), gzs.data_ptr(), ctx.hs.data_ptr(), scale.data_ptr(),
+                 gh.data_ptr(), gw.data_ptr() if gw is not None else None, ctx.n_rows, n_src, B, int(pair), cw.data_ptr(),
                  gwpart.data_ptr() if gwpart is not None else None, scratch.data_ptr(), _stream(gz))
         else:
             gzt = torch.empty(max(ctx.n_rows * B, 1), device=h.device)       # gathered tiled, as in the forward

@@ -287,6 +287,12 @@ void fh_spmm_bwd_h(const int* wave, int nwave, const int* seg, int nseg, const i
                    const int* pcol, const int* pidx, long long npos, const float* w, const void* gzs, const void* hs,
                    const float* scale, float* gh, float* gw, int n_rows, int n_src, int B, void* cw, float* gwpart,
                    float* scratch, void* stream);
+/* The same with pair: 0 as above, else two tiles per workgroup (for graphs whose gathers few rows take); gwpart then
+ * holds npos * ceil(ceil(B/64)/2) floats, and gw sums a pair's products first. */
+void fh_spmm_bwd_h_pair(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
+                        const int* pcol, const int* pidx, long long npos, const float* w, const void* gzs,
+                        const void* hs, const float* scale, float* gh, float* gw, int n_rows, int n_src, int B, int pair,
+                        void* cw, float* gwpart, float* scratch, void* stream);
 
 #ifdef __cplusplus
 }
