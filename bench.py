@@ -607,9 +607,9 @@ def hophip_leg(s, params, steps: int, warmup: int, B: int = 4096) -> dict:
             f(obs)
 
     res = {"batch": B, "workload": "FlyActor forward / teaching step (KL, autograd backward, torch.optim.Adam) with "
-                                   "its hop products on HopHip (float32: fh_to_tiled copies into fh_spmm_tiled / fh_spmm_bwd_tiled; "
-                                   "binary16 states: fh_spmm_h / fh_spmm_bwd_h) and float32 activations on FireHip "
-                                   "(fh_fire / fh_fire_bwd), states [rows][B]"}
+                                   "its layers on HopHip (float32: tiled states through fh_layer / fh_layer_bwd; binary16 states: "
+                                   "fh_spmm_h / fh_spmm_bwd_h_pair, states [rows][B] between) and float32 activations on "
+                                   "FireHip (fh_fire_tiled / fh_fire_bwd_tiled)"}
     for kernel in ("hip", "cuda16"):
         f.kernel = kernel
         out = {}

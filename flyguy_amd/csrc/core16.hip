@@ -44,7 +44,7 @@ __device__ __forceinline__ void ldf8(const float* p, float (&f)[8]) {
 
 // The products of the hop kernels: acc[k] += w_a g_a[k] + w_b g_b[k] over the lane's 8 samples, for two edges a, b
 // at once on v_dot2_f32_bf16 (two exact products and the sum in float32).  The weights come packed as bfloat16
-// values in float32 (low halves zero, k_pack<true>); v_perm_b32 pairs the two edges' weights, and the two gathered
+// values in float32 (low halves zero, k_derive<true>); v_perm_b32 pairs the two edges' weights, and the two gathered
 // states sample by sample.
 __device__ __forceinline__ void fma_pair(float wa, float wb, const u32x4& ga, const u32x4& gb, float (&acc)[8]) {
     typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
