@@ -62,7 +62,8 @@ __global__ __launch_bounds__(WG) void k_pack(const int* __restrict__ pcol, const
     if (pb == 6) {                              // (Plan::pb) the weight plane, then the source plane of the step
         unsigned char* blk = reinterpret_cast<unsigned char*>(cw) + (size_t)(p >> 6) * 384;
         reinterpret_cast<float*>(blk)[p & 63] = v;
-        reinterpret_cast<unsigned short*>(blk + 256)[p & 63] = i >= 0 ? (unsigned short)pcol[p] : (unsigned short)0xFFFF;
+        const unsigned c = i >= 0 ? (unsigned)pcol[p] : 0xFFFFu;         // (16 bits name no row past 0xFFFF: reads zeros)
+        reinterpret_cast<unsigned short*>(blk + 256)[p & 63] = (unsigned short)(c < 0xFFFFu ? c : 0xFFFFu);
         return;
     }
     cw[p] = i >= 0 ? make_int2(pcol[p], __float_as_int(v)) : make_int2(NO_ROW, 0);

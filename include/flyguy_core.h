@@ -209,7 +209,8 @@ void fh_spmm_bwd(const int* wave, int nwave, const int* seg, int nseg, const int
 /* out[B/32][rows][32] = x[rows][B] (B % 32 == 0): the layout fh_spmm_tiled and fh_spmm_bwd_tiled read. */
 void fh_to_tiled(const float* x, int rows, int B, float* out, void* stream);
 
-/* fh_spmm with the states ht tiled (fh_to_tiled); out stays [n_rows][B] row-major.  Arguments as fh_spmm. */
+/* fh_spmm with the states ht tiled (fh_to_tiled); out stays [n_rows][B] row-major.  Arguments as fh_spmm.  In all of
+ * these products a pcol entry that is no row of the states adds nothing. */
 void fh_spmm_tiled(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
                    const int* pcol, const int* pidx, long long npos, const float* w, const float* ht, float* out,
                    int n_rows, int n_src, int B, void* cw, float* scratch, void* stream);
