@@ -210,7 +210,8 @@ void fh_spmm_bwd(const int* wave, int nwave, const int* seg, int nseg, const int
 void fh_to_tiled(const float* x, int rows, int B, float* out, void* stream);
 
 /* fh_spmm with the states ht tiled (fh_to_tiled); out stays [n_rows][B] row-major.  Arguments as fh_spmm.  In all of
- * these products a pcol entry that is no row of the states adds nothing. */
+ * these products a pcol entry past the states' rows (below 2^25) reads zeros.  A plan's waves start at multiples of 64
+ * positions, as fc_plan_rows makes them: a product on tiled or binary16 states may leave out a wave that does not. */
 void fh_spmm_tiled(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
                    const int* pcol, const int* pidx, long long npos, const float* w, const float* ht, float* out,
                    int n_rows, int n_src, int B, void* cw, float* scratch, void* stream);

@@ -101,3 +101,24 @@ def test_a_source_past_the_states_reads_zeros(gpu_lib, graph, half):
     want = _forward_c(d, silent, h, half)
     got = _forward_c(dict(d, pcol=pcol), w, h, half)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_a_wave_off_the_steps_boundary_is_no_wave(gpu_lib, graph, half):
+    """The positions of a wave start at a multiple of 64 (fc_plan_rows); with 6-byte pairs a record that says otherwise
+    is refused like any other outside the plan: its rows are left alone, no other step's pairs are summed into them."""
+    index, _, w, p = graph
+    d = dict(_plan(index[0], index[1], None, w.numel()))               # (not dealt out anew: wave 0 has the longest rows)
+    h, _ = _states(64, 4)
+    last = len(p["wave"]) - 1
+    while p["wave"][last, 1] == 0:
+        last -= 1
+    wave = d["wave"].clone()
+    wave[last, 0] -= 32
+    touched = p["seg"][8 * last:8 * last + 8]
+    touched = put(touched[(touched[:, 0] >= 0) & (touched[:, 1] < 0), 0], np.int64)
+    want = _forward_c(d, w, h, half)
+    got = _forward_c(dict(d, wave=wave), w, h, half)
+    assert len(touched) and (got[touched] == 7).all()
+    want[touched] = 7
+    assert torch.equal(got, want)
