@@ -138,7 +138,7 @@ struct Core {
     std::vector<unsigned char*> fire_bytes;
     std::vector<unsigned*> fire_bits;
     long long adam_t = 0;
-    int B = 0;
+    int n = 0;                       // the last forward's samples (those that fill its last tile repeat the last one)
     hipStream_t st = nullptr;
     std::vector<void*> allocs;
     Prof prof;

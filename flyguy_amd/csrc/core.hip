@@ -886,7 +886,7 @@ bool forward(Core& c, const float* obs, int B, float* logits, int set, int n) {
         FG_CHECK(launch_logits_mfma(hp, false, c.sizes[c.hops], c.dn, c.n_dn, c.arr(set, 6), c.n_act, c.owT, c.lpart, logits,
                                     B, n, st), false);
     }
-    c.B = B;
+    c.n = n;
     return true;
 }
 
@@ -1039,7 +1039,7 @@ static bool forward16(Core& c, const float* obs, int B, float* logits, int set, 
         FG_CHECK(launch_logits_mfma(hp, true, c.sizes[c.hops], c.dn, c.n_dn, c.arr(set, 6), c.n_act, c.owT, c.lpart, logits,
                                     B, n, st), false);
     }
-    c.B = B;
+    c.n = n;
     return true;
 }
 
@@ -1286,7 +1286,7 @@ void fc_backward_n(void* h, const float* dlogits, int n) {
     const int B = ragged_batch(c, n);
     if (!B) return;
     if (!dlogits) { set_error("fc_backward_n: null pointer"); return; }
-    if (B != c->B) { set_error("fc_backward_n: batch differs from the last forward's"); return; }
+    if (n != c->n) { set_error("fc_backward_n: batch differs from the last forward's"); return; }
     if (n < B) {
         FG_CHECK(launch_pad(dlogits, (long long)n * c->n_act, c->dl, (long long)B * c->n_act, c->st), );
         dlogits = c->dl;
@@ -1305,7 +1305,7 @@ void fc_backward(void* h, const float* dlogits, int B) {
     Core* c = (Core*)h;
     if (!check_batch(c, B)) return;
     if (!dlogits) { set_error("fc_backward: null pointer"); return; }
-    if (B != c->B) { set_error("fc_backward: batch differs from the last forward's"); return; }
+    if (B != c->n) { set_error("fc_backward: batch differs from the last forward's"); return; }
     backward(*c, dlogits, B);
 }
 

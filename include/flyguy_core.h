@@ -45,7 +45,8 @@ void fc_forward(void* core, const float* obs, int B, float* logits, int ema);
 
 /* fc_forward and fc_backward for any number of samples, n >= 1, that rounded up to whole tiles (32 samples, 64 with
  * bfloat16 states) is at most max_batch: obs [n][obs_dim], logits and dlogits [n][n_act].  The samples that fill the
- * last tile repeat the last one and have no gradient.  Same results as the padded calls, without the copies. */
+ * last tile repeat the last one and have no gradient: n of fc_backward_n, and B of fc_backward, are the last forward's
+ * number of samples.  Same results as the padded calls, without the copies. */
 void fc_forward_n(void* core, const float* obs, int n, float* logits, int ema);
 void fc_backward_n(void* core, const float* dlogits, int n);
 

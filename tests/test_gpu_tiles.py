@@ -168,3 +168,26 @@ def test_any_number_of_samples(gpu_lib, net, n, bf16):
     for bad in (0, -1, 129, 2**31 - 1):
         with pytest.raises(RuntimeError):
             call("fc_forward_n", core.h, x.data_ptr(), bad, logits.data_ptr(), 0)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_a_gradient_of_another_batch_is_refused(gpu_lib, net, bf16):
+    """fc_backward_n takes the last forward's number of samples and fc_backward a batch that was whole: the samples that
+    filled the last tile have no gradient, and no real one is left out."""
+    s, params = net
+    core = Core(s, params, 128, int(bf16))
+    x = torch.randn(128, s["obs_dim"], device="cuda", generator=torch.Generator(device="cuda").manual_seed(0))
+    d = torch.ones(128, s["n_act"], device="cuda")
+    logits = torch.empty(128, s["n_act"], device="cuda")
+    core.zero_grad()
+    call("fc_forward_n", core.h, x.data_ptr(), 100, logits.data_ptr(), 0)
+    for name, n in (("fc_backward_n", 99), ("fc_backward_n", 101), ("fc_backward_n", 128), ("fc_backward", 128)):
+        with pytest.raises(RuntimeError):
+            call(name, core.h, d.data_ptr(), n)
+    assert not any(g.any() for g in core.get(4))
+    call("fc_backward_n", core.h, d.data_ptr(), 100)
+    call("fc_forward", core.h, x.data_ptr(), 128, logits.data_ptr(), 0)
+    with pytest.raises(RuntimeError):
+        call("fc_backward_n", core.h, d.data_ptr(), 100)
+    call("fc_backward", core.h, d.data_ptr(), 128)
+    call("fc_backward_n", core.h, d.data_ptr(), 128)
