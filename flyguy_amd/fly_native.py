@@ -99,8 +99,8 @@ class _Session:
     def evaluate(self, obs: torch.Tensor, n_act: int) -> torch.Tensor:
         """Logits of one piece (at most max_batch samples; the library fills the last tile with its last row)."""
         n = obs.shape[0]
-        if obs.numel() < n * self.obs_dim or (obs.dim() != 2 and n % TILE):
-            raise ValueError("NativeFlyActor: observations must be [samples, obs_dim]")
+        if obs.numel() != n * self.obs_dim:
+            raise ValueError("NativeFlyActor: observations must hold obs_dim values a sample")
         x = obs.contiguous()
         logits = torch.empty(n, n_act, device=x.device)
         self.on_current_stream(x.device)
