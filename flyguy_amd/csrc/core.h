@@ -124,7 +124,8 @@ struct Core {
     };
     unsigned long long wver[2] = {1, 1};
     // Whether the gradient entries that no backward writes (neurons and strengths out of play, the arrays' padding) are
-    // zero: until a gradient is copied in.  A step whose backward stores every other entry (fresh) clears nothing then.
+    // zero: until a gradient is copied in, and again once a clearing ran (not one only recorded into a graph).  A step
+    // whose backward stores every other entry (fresh) clears nothing then.
     bool grad_rest_zero = true;
     // The tables in the order of their jobs (DeriveJob), each group a run of blocks: group g's are [dblock[g], dblock[g + 1])
     enum Table { T_FPAIRS = 0, T_INFO = 1, T_OWT = 2, T_TPAIRS = 3, T_COUNT = 4 };
@@ -193,7 +194,10 @@ bool backward(Core& c, const float* dlogits, int B, bool fresh = false);
 // the backward's (from the weights, so with bwd the set is SET_P).  forward() and backward() call it for their own; a
 // step that runs both calls it for both first, in one launch.
 bool derive(Core& c, int set, bool fwd, bool bwd);
-// Ahead of a fresh backward: clears the gradient, unless what that backward does not store is zero already
+// Clears the gradient
+bool clear_grad(Core& c);
+// Ahead of a fresh backward: clears the gradient, unless what that backward does not store is zero already.  A step
+// recorded into a graph always clears: a gradient may be copied in before any replay.
 bool clear_for_fresh(Core& c);
 float grad_norm(Core& c);
 // Adam + running average over all seven arrays; lr for W, lr_neuron for gain / theta, lr_plug for the rest

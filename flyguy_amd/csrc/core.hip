@@ -1134,12 +1134,24 @@ static bool backward16(Core& c, const float* dlogits, int B, bool fresh) {
     return true;
 }
 
-bool clear_for_fresh(Core& c) {
-    if (c.grad_rest_zero) return true;
-    Timed t(c, ST_ZERO);
-    FG_CHECK(launch_fill(c.arr(SET_G, 0), 0.f, c.PT, c.st), false);
-    c.grad_rest_zero = true;
+// whether the stream records its work into a graph (or cannot say) instead of running it
+static bool recording(hipStream_t st) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
     return true;
+}
+
+bool clear_grad(Core& c) {
+    FG_CHECK(launch_fill(c.arr(SET_G, 0), 0.f, c.PT, c.st), false);
+    if (!recording(c.st)) c.grad_rest_zero = true;
+    return true;
+}
+
+bool clear_for_fresh(Core& c) {
+    if (c.grad_rest_zero && !recording(c.st)) return true;
+    Timed t(c, ST_ZERO);
+    return clear_grad(c);
 }
 
 float grad_norm(Core& c) {
@@ -1297,8 +1309,7 @@ void fc_backward_n(void* h, const float* dlogits, int n) {
 void fc_zero_grad(void* h) {
     Core* c = (Core*)h;
     if (!c) { set_error("null handle"); return; }
-    FG_CHECK(launch_fill(c->arr(SET_G, 0), 0.f, c->PT, c->st), );
-    c->grad_rest_zero = true;
+    clear_grad(*c);
 }
 
 void fc_backward(void* h, const float* dlogits, int B) {

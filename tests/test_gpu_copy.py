@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from flyguy_amd._lib import LibraryError, call
+from flyguy_amd._lib import LibraryError, call, lib
 from flyguy_amd.synth import scaled_3hop
 from gpu_helpers import NAMES, Core
 
@@ -77,3 +77,63 @@ def test_step_after_a_copied_gradient(gpu_lib, bf16):
     for name, a, b in zip(NAMES, *got):
         assert np.array_equal(a, b), name
     assert not got[0][1][-5:].any() and not got[0][2][-5:].any()
+
+
+def _lone_neurons():
+    """A network with five neurons in no layer, whose gradient entries no backward writes, and a batch for it."""
+    s, params = scaled_3hop(64)
+    s = dict(s, n_neurons=s["n_neurons"] + 5)
+    params = list(params)
+    params[1] = np.concatenate([params[1], np.ones(5, np.float32)])
+    params[2] = np.concatenate([params[2], np.zeros(5, np.float32)])
+    rng = np.random.default_rng(0)
+    return s, params, *(torch.as_tensor(rng.standard_normal((64, n)).astype(np.float32)).cuda()
+                        for n in (s["obs_dim"], s["n_act"]))
+
+
+def _step(core, obs, tl):
+    call("fc_teach_step", core.h, obs.data_ptr(), tl.data_ptr(), 64, 1.0, 0.0, 0.0, 0.0, 0.0, 0.9, None)
+
+
+def test_a_captured_step_clears_what_was_copied_in_since(gpu_lib):
+    """A teaching step in a HIP graph (its rates zero, so that every replay sees the same weights), with a gradient
+    copied in before each replay: the eager step's gradient every time."""
+    s, params, obs, tl = _lone_neurons()
+    core = Core(s, params, 64)
+    _step(core, obs, tl)
+    want = core.get(4)
+    stream = torch.cuda.Stream()
+    lib().fc_set_stream(core.h, stream.cuda_stream)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        _step(core, obs, tl)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        _step(core, obs, tl)
+    for i in range(3):
+        core.set(4, [np.full(n, 3.0 + i, np.float32) for n in core.sizes])
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, a, b in zip(NAMES, want, core.get(4)):
+            assert np.array_equal(a, b), (i, name)
+
+
+def test_a_captured_clearing_has_cleared_nothing_yet(gpu_lib):
+    """fc_zero_grad recorded into a graph that has not run: the next step still clears the gradient copied in before."""
+    s, params, obs, tl = _lone_neurons()
+    core = Core(s, params, 64)
+    _step(core, obs, tl)
+    want = core.get(4)
+    core.set(4, [np.full(n, 3.0, np.float32) for n in core.sizes])
+    stream = torch.cuda.Stream()
+    lib().fc_set_stream(core.h, stream.cuda_stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        core.zero_grad()
+    lib().fc_set_stream(core.h, 0)
+    _step(core, obs, tl)
+    for name, a, b in zip(NAMES, want, core.get(4)):
+        assert np.array_equal(a, b), name
