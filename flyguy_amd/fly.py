@@ -365,7 +365,7 @@ class FlyActor(nn.Module):
         if self.kernel != "torch" and obs.is_cuda and obs.shape[0] % 32 == 0:      # (at any batch size)
             from .fly_hip import FireHip, HopHip
             half = self.kernel == "cuda16"
-            if not half and self.w.dtype == torch.float32 and obs.shape[0]:
+            if not half and self.w.dtype == self.in_b.dtype == torch.float32 and obs.shape[0]:
                 return self._walk_tiled(obs)
 
             def on_library(k, layer, w, h):

@@ -70,3 +70,27 @@ def test_actor_gradients_through_the_library(gpu_lib, hops):
     for (name, p), (_, q) in zip(g.named_parameters(), ref.named_parameters()):
         assert p.grad is not None, name
         assert rel(p.grad.double().cpu().numpy(), q.grad.numpy()) <= 1e-4, name
+
+
+@pytest.mark.parametrize("name", ["in_b", "gain", "theta", "in_w"])
+def test_an_array_of_another_type_is_widened(gpu_lib, name):
+    """An actor whose strengths are float32 and one other array is held in binary16: logits as with that array's values in
+    float32, and a gradient in the array's own type."""
+    torch.manual_seed(3)
+    f = lively(FlyActor(toy("b"), 517, 90, hops=3, fan=16)).cuda()
+    f.kernel = "hip"
+    x = torch.randn(64, 517, device="cuda")
+    p = getattr(f, name)
+    p.data = p.data.half().float()
+    want = f(x)
+    want.square().mean().backward()
+    grad, p.grad = p.grad, None
+    p.data = p.data.half()
+    got = f(x)
+    got.square().mean().backward()
+    # theta: softplus itself is taken in binary16, half a unit of 2^-11 of thresholds below 1 and their effect on logits
+    # of the order of one
+    tol = 1e-2 if name == "theta" else 1e-5
+    assert rel(got.detach().cpu(), want.detach().cpu()) <= tol
+    assert p.grad.dtype == torch.float16
+    assert rel(p.grad.float().cpu(), grad.cpu()) <= max(tol, 2.0 ** -10)
