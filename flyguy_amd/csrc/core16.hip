@@ -112,7 +112,7 @@ __global__ __launch_bounds__(WG) void k_cfwd16(Plan p, const int2* __restrict__ 
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = wave_of(p, rb, RB);
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(WG) void k_cbwd16(Plan p, const int2* __restrict__ 
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(WG) void k_cbwd16x2(Plan p, const int2* __restrict_
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;

@@ -50,13 +50,14 @@ __device__ __forceinline__ int wave_of(const Plan& p, int rb, int RB) {
 }
 
 // wave w of the plan ({woff, longest segment}); false when w is past the end, names positions outside the plan or, with
-// 6-byte pairs, which are stored by blocks of 64 positions, starts inside a block
+// 6-byte pairs (PB 6), which are stored by blocks of 64 positions, starts inside a block
+template <int PB>
 __device__ __forceinline__ bool load_wave(const Plan& p, int w, int2& wv) {
     wv = make_int2(0, 0);
     if (w >= p.nwave) return false;
     const int2 v = p.wave[w];
-    if (v.x < 0 || v.y < 0 || (long long)v.x + 64 * (((long long)v.y + 7) / 8) > p.npos) return false;
-    if (p.pb == 6 && (v.x & 63)) return false;
+    constexpr int bad = PB == 6 ? (int)0x8000003Fu : (int)0x80000000u;    // (the sign bit: x < 0)
+    if ((v.x & bad) != 0 || v.y < 0 || (long long)v.x + 64 * (((long long)v.y + 7) / 8) > p.npos) return false;
     wv = v;
     return true;
 }

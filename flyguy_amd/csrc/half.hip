@@ -101,7 +101,7 @@ __global__ __launch_bounds__(WG) void k_fwd16(Plan p, const int2* __restrict__ c
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(WG) void k_bwd16(Plan p, const int2* __restrict__ c
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(WG) void k_bwd16x2(Plan p, const int2* __restrict__
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;

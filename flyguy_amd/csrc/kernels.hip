@@ -183,7 +183,7 @@ __global__ __launch_bounds__(WG) void k_fwd(Plan p, const int2* __restrict__ cw,
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = wave_of(p, rb, RB);
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(64) void k_fwd_deep(Plan p, const int2* __restrict_
     if (w >= p.nwave) return;
     const int lane = threadIdx.x, grp = lane >> 3, sub = lane & 7;
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const int steps = wok ? (wv.y + 7) / 8 : 0;
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt[U];
@@ -717,7 +717,7 @@ __global__ __launch_bounds__(WG) void k_bwd(Plan p, const int2* __restrict__ cw,
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;
@@ -786,7 +786,7 @@ __global__ __launch_bounds__(WG) void k_bwd2(Plan p, const int2* __restrict__ cw
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(rb * (WG / 64) + (int)(threadIdx.x >> 6));
     int2 wv;
-    const bool wok = load_wave(p, w, wv);
+    const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);
     int2 nxt = (wok && wv.y > 0) ? q.step(0) : make_int2(NO_ROW, 0);
     int4 sg;
