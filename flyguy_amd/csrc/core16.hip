@@ -97,6 +97,13 @@ __device__ __forceinline__ void fwd_finish16(const FwdEpi16& e, int t, int tile,
     }
 }
 
+// A striped plan (Plan::stripe) is taken in a row on a tile whose source layer has a sixth of its rows silent.  Hop 1 / 2
+// of the benchmark network at 128 tiles, striped and in a row, us: no row silenced 1105 / 1421 and 1138 / 1457 (9% of hop
+// 2's rows are silent by themselves); a tenth of all neurons 1171 / 1334 and 1166 / 1344; a fifth 1151 / 1280 and 1126 /
+// 1255; a quarter 1144 / 1258 and 1106 / 1221; half 1121 / 1214 and 1059 / 1153.  (In float32, twice the gathers for the
+// same sums, striped is faster throughout: a quarter 986 / 1100 and 1011 / 1129, half 933 / 1027 and 952 / 1056.)
+constexpr int SILENT_IN_A_ROW = 6;
+
 // the plug or one hop over its row plan (as k_fwd); split rows leave float32 partials [T][nslot][64]
 // src_fires: the source layer's firing bitmaps (k_fires_pack, fw_ld words per tile; fw_ld 0: none)
 template <int PB>
@@ -108,9 +115,10 @@ __global__ __launch_bounds__(WG) void k_cfwd16(Plan p, const int2* __restrict__ 
     int rb;
     const int tile = tile_of(blockIdx.x, RB, T, rb, p.stripe);
     if (rb >= RB) return;
-    const bool bits = stage_fires(src_fires, fw_ld, tile, fires);     // (only for a tile with silent source rows)
+    int silent = 0;
+    const bool bits = stage_fires(src_fires, fw_ld, tile, fires, &silent);     // (only for a tile with silent source rows)
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
-    const int w = wave_of(p, rb, RB);
+    const int w = wave_of(rb, RB, p.stripe && SILENT_IN_A_ROW * silent < src_rows);
     int2 wv;
     const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);

@@ -42,11 +42,10 @@ __device__ __forceinline__ float dot4(const float4& a, const float4& b) {
 }
 __device__ __forceinline__ float hsum4(const float4& a) { return ((a.x + a.y) + a.z) + a.w; }
 
-// the plan wave of this wave of row block rb (of RB blocks): four in a row, or (Plan::stripe) one from each quarter of
-// the plan
-__device__ __forceinline__ int wave_of(const Plan& p, int rb, int RB) {
+// the plan wave of this wave of row block rb (of RB blocks): four in a row, or (stripe) one from each quarter of the plan
+__device__ __forceinline__ int wave_of(int rb, int RB, bool stripe) {
     const int i = (int)(threadIdx.x >> 6);
-    return __builtin_amdgcn_readfirstlane(p.stripe ? rb + RB * i : rb * (WG / 64) + i);
+    return __builtin_amdgcn_readfirstlane(stripe ? rb + RB * i : rb * (WG / 64) + i);
 }
 
 // wave w of the plan ({woff, longest segment}); false when w is past the end, names positions outside the plan or, with
@@ -137,11 +136,14 @@ __device__ __forceinline__ bool bf16_lane_fires(const u32x4& h) {
     return ((h[0] | h[1] | h[2] | h[3]) & 0x7FFF7FFFu) != 0u;
 }
 // Stage the firing bitmap of a tile (k_fires_pack) in LDS when the tile has silent rows; every thread of the
-// workgroup calls this.  Returns whether it did (then the hop skips the silent rows' gathers).
-__device__ __forceinline__ bool stage_fires(const unsigned* src_fires, int fw_ld, int tile, unsigned* lds) {
+// workgroup calls this.  Returns whether it did (then the hop skips the silent rows' gathers); silent: how many there are.
+__device__ __forceinline__ bool stage_fires(const unsigned* src_fires, int fw_ld, int tile, unsigned* lds,
+                                            int* silent = nullptr) {
     if (fw_ld <= 0) return false;
     const unsigned* b = src_fires + (size_t)tile * fw_ld;
-    if (__builtin_amdgcn_readfirstlane(b[0]) == 0) return false;     // (uniform: one word for the whole workgroup)
+    const int n = __builtin_amdgcn_readfirstlane(b[0]);              // (uniform: one word for the whole workgroup)
+    if (n == 0) return false;
+    if (silent) *silent = n;
     const uint4* b4 = reinterpret_cast<const uint4*>(b + 4);
     for (int i = threadIdx.x; i < (fw_ld - 4) / 4; i += WG) reinterpret_cast<uint4*>(lds)[i] = b4[i];
     __syncthreads();

@@ -41,7 +41,8 @@ struct Plan {
     int nslot = 0;
     long long npos = 0;
     int pb = 8;
-    bool stripe = false;              // k_fwd, k_cfwd16: a workgroup takes a wave from each quarter of the plan
+    bool stripe = false;              // k_fwd, k_cfwd16: a workgroup takes a wave from each quarter of the plan (k_cfwd16:
+                                      //   not on a tile of many silent rows)
 };
 // the bytes the pairs of npos positions take
 inline long long pair_bytes(long long npos, int pb) { return npos * (pb == 6 ? 6 : 8); }

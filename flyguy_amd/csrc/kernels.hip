@@ -181,7 +181,7 @@ __global__ __launch_bounds__(WG) void k_fwd(Plan p, const int2* __restrict__ cw,
     if (rb >= RB) return;
     const bool bits = stage_fires(src_fires, fw_ld, tile, fires);     // (only for a tile with silent source rows)
     const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7, lane = threadIdx.x & 63;
-    const int w = wave_of(p, rb, RB);
+    const int w = wave_of(rb, RB, p.stripe);
     int2 wv;
     const bool wok = load_wave<PB>(p, w, wv);
     const PairLoad<PB> q(cw, wv.x, lane);

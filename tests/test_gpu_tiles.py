@@ -191,3 +191,22 @@ def test_a_gradient_of_another_batch_is_refused(gpu_lib, net, bf16):
         call("fc_backward_n", core.h, d.data_ptr(), 100)
     call("fc_backward", core.h, d.data_ptr(), 128)
     call("fc_backward_n", core.h, d.data_ptr(), 128)
+
+
+@pytest.mark.parametrize("share", [0.0, 0.1, 0.3, 0.9])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_order_of_waves_over_silent_rows(gpu_lib, uneven, monkeypatch, bf16, share):
+    """A plan of unequal rows is walked in one order or another by the share of silent source rows: logits and every
+    layer's states bit for bit those of a forward that skips none."""
+    s, params = uneven
+    params = list(params)
+    params[2] = np.where(np.random.default_rng(1).random(params[2].size) < share, np.float32(30), params[2]).astype(np.float32)
+    B = 64 * 11
+    obs = np.random.default_rng(2).standard_normal((B, s["obs_dim"])).astype(np.float32)
+    got = []
+    for mode in ("0", "1"):
+        monkeypatch.setenv("FLYGUY_SKIP_SILENT", mode)
+        core = Core(s, params, B, int(bf16))
+        got.append([core.forward(obs)] + [core.state(k, 0, n, B) for k, n in enumerate(s["sizes"])])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
