@@ -809,15 +809,19 @@ static int plug_split(const Core& c, int T, int total = 2048) {
     return T >= 64 ? std::max(1, total / T) : 0;
 }
 
-// Whether a hop's forward skips the gathers of silent source rows: the layer below then records a byte per row and a
-// launch packs them (k_fires_pack, 5 us), and on the benchmark network (8.9% silent lines) hop 2 gains 7%.  So from
-// FIRES_MIN_LINES gathered lines (about 90 us) up, and never in a launch of few tiles (fwd_deep).  Forward without /
-// with bitmaps at 6, 8, 13, 16, 32 tiles: 205 / 213, 233 / 243, 362 / 366, 417 / 422, 807 / 797 us; hop 2 alone with them
-// from 8 tiles up: 13 tiles 357, 16 tiles 414 us.  FLYGUY_SKIP_SILENT=1 takes them at every batch.
-constexpr long long FIRES_MIN_LINES = 12000000;
-static bool fwd_skips(const Core& c, const HopD& d, int T, bool bf16) {
+// Whether a hop's forward skips the gathers of silent source rows.  The layer below then records a byte per row and a
+// launch packs them: 7 to 13 us, whatever they save.  So from FIRES_MIN_LINES gathered lines up, where what a quarter of
+// the rows silent saves (a trained network's share: 22 to 28%) and what it costs where none is are about alike.  Forward
+// of the benchmark network (hops of 1.2, 1.5 and 0.29 million lines a tile) / of the Erdos-Renyi one, us without and with
+// the skips that the line at 7 instead of 12 million adds:
+//   a quarter silent: 6 tiles 199 -> 175 / 178 -> 164, 24 tiles 539 -> 528 / 515 -> 509, 33 tiles 774 -> 752 / 707 -> 694;
+//   none silenced:    6 tiles 199 -> 200 / 178 -> 187, 24 tiles 604 -> 612 / 615 -> 627, 33 tiles 854 -> 860 / 840 -> 852;
+// at 6 million lines 4 tiles lose 5% with none silent and 1% with a quarter.  bfloat16, 24 and 32 tiles: a quarter
+// silent 613 -> 597 and 796 -> 778, none 654 -> 659 and 843 -> 849.  FLYGUY_SKIP_SILENT=1 takes them at every batch.
+constexpr long long FIRES_MIN_LINES = 7000000;
+static bool fwd_skips(const Core& c, const HopD& d, int T) {
     if (!c.skip_silent || c.skip_always) return c.skip_silent;
-    return (long long)d.E * T >= FIRES_MIN_LINES && (bf16 || !fwd_deep(d.fp.view(), T));
+    return (long long)d.E * T >= FIRES_MIN_LINES;
 }
 
 bool forward(Core& c, const float* obs, int B, float* logits, int set, int n) {
@@ -831,7 +835,7 @@ bool forward(Core& c, const float* obs, int B, float* logits, int set, int n) {
     c.tables_old = true;
     // a layer whose next hop skips its silent rows records which rows fire on each tile, packed into bitmaps before that
     // hop
-    auto skips = [&](int layer) { return layer < c.hops && fwd_skips(c, c.hop[(size_t)layer], T, false); };
+    auto skips = [&](int layer) { return layer < c.hops && fwd_skips(c, c.hop[(size_t)layer], T); };
     auto bytes = [&](int layer) { return skips(layer) ? c.fire_bytes[(size_t)layer] : nullptr; };
     auto bits = [&](int layer) { return skips(layer) ? c.fire_bits[(size_t)layer] : nullptr; };
     FwdEpi e0;
@@ -996,7 +1000,7 @@ static bool forward16(Core& c, const float* obs, int B, float* logits, int set, 
     hipStream_t st = c.st;
     { Timed t(c, ST_OBS); FG_CHECK(launch_obs_in16(obs, s16(c.x), c.obs_dim, B, n, st), false); }
     if (!derive(c, set, true, false)) return false;
-    auto skips = [&](int layer) { return layer < c.hops && fwd_skips(c, c.hop[(size_t)layer], T, true); };   // (as forward)
+    auto skips = [&](int layer) { return layer < c.hops && fwd_skips(c, c.hop[(size_t)layer], T); };   // (as forward)
     auto bytes = [&](int layer) { return skips(layer) ? c.fire_bytes[(size_t)layer] : nullptr; };
     auto bits = [&](int layer) { return skips(layer) ? c.fire_bits[(size_t)layer] : nullptr; };
     FwdEpi16 e0;
