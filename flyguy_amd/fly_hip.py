@@ -30,6 +30,14 @@ _plans: OrderedDict = OrderedDict()
 _checked: OrderedDict = OrderedDict()
 _CACHE = 64
 
+# The tiled and binary16 backwards take two tiles per workgroup where the core's does (bwd_pairs), from this many samples
+# up.  Hops 1 / 2 of the benchmark network, one and two tiles, us: binary16 at B=192 129 / 150 and 138 / 161, B=256 141 /
+# 166 and 142 / 167, B=512 184 / 228 and 185 / 221; float32 at B=96 88 / 111 and 95 / 123, B=256 124 / 159 and 128 / 168,
+# B=512 185 / 266 and 191 / 254.  The strengths' gradient, a pair's products added before the rest, is off its float64
+# value by 6.27e-8 (one tile: 6.17e-8) with the two binary16 tiles of B=128, 6.85e-8 (6.89e-8) at B=256, 7.48e-8 (7.90e-8)
+# at B=512 and less than one tile's from there on.
+PAIR_FROM = 512
+
 
 def available() -> bool:
     """True when a GPU is present and the library loads (a missing library on a GPU is an error, not False)."""
@@ -212,7 +220,7 @@ class HopHip(torch.autograd.Function):
             call("fh_absmax", gz.data_ptr(), gz.numel(), scale.data_ptr(), _stream(gz))
             gzs = torch.empty(max(t64 * ctx.n_rows * 64, 1), dtype=torch.float16, device=h.device)
             call("fh_to_half", gz.data_ptr(), ctx.n_rows, B, scale.data_ptr(), gzs.data_ptr(), _stream(gz))
-            pair = ctx.pair and t64 > 1      # two tiles per workgroup where the core's backward takes two (pair_tiles)
+            pair = ctx.pair and B >= PAIR_FROM
             gwpart = torch.empty(max(d["npos"] * (-(-t64 // 2) if pair else t64), 1),
                                  device=h.device) if gw is not None else None
             scratch = torch.empty(max(d["nslot"] * t64 * 64, 1), device=h.device)
@@ -271,7 +279,7 @@ def _layer_backward(ctx, gz):
     _check_index(tcol, n_rows, "target index")
     _check_index(tperm, E, "transposed order")
     d = _plan(tcrow, tcol, tperm, E)
-    pair = ctx.pair and T > 1                # two tiles per workgroup where the core's backward takes two (pair_tiles)
+    pair = ctx.pair and B >= PAIR_FROM
     gh = torch.empty(T, n_src, 32, device=h.device)
     gw = torch.zeros_like(w) if ctx.needs_input_grad[0] else None
     cw = torch.empty(max(d["npos"], 1), 2, dtype=torch.int32, device=h.device)
