@@ -138,8 +138,8 @@ struct DeriveJob {
 };
 // the blocks a job takes
 long long derive_blocks(const DeriveJob& j);
-// Jobs [j0, j0 + n) of the table at `jobs` (device memory); first (device): each job's first block, counted from job 0;
-// b0, blocks: the first block and the number of blocks of the range.  set: the weights' set; gain, theta: its arrays.
+// A run of blocks of the table at `jobs` (device memory, njobs of them); first (device): each job's first block, counted
+// from job 0; b0, blocks: the run's first block and its length.  set: the weights' set; gain, theta: its arrays.
 // bf16w: pair weights rounded to bfloat16 (nearest even), as the float32 of that value
 hipError_t launch_derive(const DeriveJob* jobs, const int* first, int njobs, long long b0, long long blocks,
                          const float* set, const float* gain, const float* theta, bool bf16w, hipStream_t st);

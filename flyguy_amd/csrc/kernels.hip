@@ -240,6 +240,7 @@ __global__ __launch_bounds__(WG) void k_fwd(Plan p, const int2* __restrict__ cw,
 template <int PB, int U>
 __global__ __launch_bounds__(64) void k_fwd_deep(Plan p, const int2* __restrict__ cw, const float* __restrict__ src,
                                                  int src_rows, FwdEpi epi, float* __restrict__ part, Lay lp, int T) {
+    static_assert(U == 2 || U == 4, "the last steps below");
     __shared__ __align__(16) int2 slots[U][RPW][LPR];
     int w;
     const int tile = tile_of(blockIdx.x, p.nwave, T, w, p.stripe);
@@ -292,16 +293,15 @@ __global__ __launch_bounds__(64) void k_fwd_deep(Plan p, const int2* __restrict_
     };
     int j = 0;
     for (; j + U <= steps; j += U) round(std::integral_constant<int, U>{}, j);
-    if (j < steps) {                            // the last steps: the next power of two of them
-        const int r = steps - j;
-        if (r == 1)
+    if (j < steps) {                            // the last steps, fewer than U (2 or 4): the next power of two of them
+        if (steps - j == 1)
             round(std::integral_constant<int, 1>{}, j);
-        else if (r == 2)
-            round(std::integral_constant<int, 2>{}, j);
-        else if (U > 4 && r <= 4)
-            round(std::integral_constant<int, 4>{}, j);
-        else
-            round(std::integral_constant<int, U>{}, j);
+        else if constexpr (U > 2) {
+            if (steps - j == 2)
+                round(std::integral_constant<int, 2>{}, j);
+            else
+                round(std::integral_constant<int, U>{}, j);
+        }
     }
     if (steps == 0) inputs();
     if (!live) return;
