@@ -41,21 +41,8 @@ def _degrees(rng, rows: int, total: int, cap: int, sigma: float, kind: str) -> n
 
 
 def _unique_sources(rng, d: np.ndarray, n_src: int) -> tuple[np.ndarray, np.ndarray]:
-    """Row and source of every connection, sorted by (row, source), no repeated source within a row."""
-    row = np.repeat(np.arange(len(d), dtype=np.int64), d)
-    col = rng.integers(0, n_src, len(row), dtype=np.int64)
-    while True:
-        order = np.lexsort((col, row))
-        col = col[order]
-        dup = np.flatnonzero((col[1:] == col[:-1]) & (row[1:] == row[:-1])) + 1
-        if len(dup) == 0:
-            return row, col
-        col[dup] = rng.integers(0, n_src, len(dup), dtype=np.int64)
-
-
-def _unique_sources_large(rng, d: np.ndarray, n_src: int) -> tuple[np.ndarray, np.ndarray]:
-    """_unique_sources for large graphs: one sort of (row, source) keys, then only the rows that still hold a repeated
-    source are redrawn and re-sorted."""
+    """Row and source of every connection, sorted by (row, source), no repeated source within a row: one sort of (row,
+    source) keys, then only the rows that still hold a repeated source are redrawn and re-sorted."""
     row = np.repeat(np.arange(len(d), dtype=np.int64), d)
     key = row * n_src + rng.integers(0, n_src, len(row), dtype=np.int64)
     key.sort()
@@ -137,7 +124,7 @@ def whole_connectome(neurons: int = WHOLE["neurons"], connections: int = WHOLE["
     can carry the signal (its pruning, fly.py:91-121)."""
     rng = np.random.default_rng(seed)
     d = _degrees(rng, neurons, connections, neurons, sigma, "lognormal")
-    post, pre = _unique_sources_large(rng, d, neurons)
+    post, pre = _unique_sources(rng, d, neurons)
     perm = rng.permutation(connections)
     ids = rng.permutation(neurons)
     return {"body": np.arange(neurons, dtype=np.int64), "pre": pre[perm].astype(np.int32),
