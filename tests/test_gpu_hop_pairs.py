@@ -225,7 +225,7 @@ def test_pairs_of_tiles_from_a_batch_up(gpu_lib, light, monkeypatch):
 
 # ------------------------------------------------------------------------------------------------ plans of a caller's own
 def _forward_c(d, w, h, half):
-    """A caller's product through the C entry points on a plan d: (with row-major states or none, tiled or binary16)."""
+    """A product as a C caller makes it on the plan d, over tiled or binary16 states."""
     n_src, B = h.shape
     n_rows, st = HEAVY + LIGHT, torch.cuda.current_stream().cuda_stream
     cw = torch.empty(d["npos"], 2, dtype=torch.int32, device="cuda")
