@@ -127,7 +127,8 @@ __device__ __forceinline__ float4 ld_stream(const float4* p) {
     return make_float4(v.x, v.y, v.z, v.w);
 }
 // The row's own inputs of the finish (re-drive row d, gain, threshold), loaded before the edge loop so that their
-// latency hides behind the gathers.
+// latency hides behind the gathers.  (The drive is tiled: its tile holds tile / TW rows, and a field of a caller's plan
+// that names none of them reads no drive.)
 struct FwdIn {
     float4 dv;
     float g, sp, b;                             // b: the row's bias (the plug's records carry it)
@@ -136,7 +137,7 @@ struct FwdIn {
 // the row for a split one; nullptr: none)
 __device__ __forceinline__ FwdIn fwd_inputs(const FwdEpi& e, const float4* recs, int i, int d, int tile, int sub) {
     FwdIn in{make_float4(0.f, 0.f, 0.f, 0.f), 0.f, 0.f, 0.f};
-    if (e.drive && d >= 0) in.dv = ld_stream(at4u(e.drive, e.ldrive, tile, d, sub));
+    if (e.drive && (unsigned)d < (unsigned)e.ldrive.tile / TW) in.dv = ld_stream(at4u(e.drive, e.ldrive, tile, d, sub));
     if (recs) {
         const float4 r = recs[i];
         in.g = r.x;

@@ -228,8 +228,8 @@ void fh_spmm_bwd_tiled(const int* wave, int nwave, const int* seg, int nseg, con
  * reference ---- */
 
 /* out (tiled, n_rows) = A ht, each row's sum plus bias[row] (null: none) and plus row d of drive (tiled, n_s rows; null:
- * none) where the row's re-drive field in the plan is d >= 0 (third int of a segment, fourth of a split row; -1 none,
- * below n_s).  Other arguments as fh_spmm_tiled. */
+ * none) where the row's re-drive field in the plan is d (third int of a segment, fourth of a split row; -1, or any d that
+ * is no row of the drive: none).  Other arguments as fh_spmm_tiled. */
 void fh_layer(const int* wave, int nwave, const int* seg, int nseg, const int* split, int nsplit, int nslot,
               const int* pcol, const int* pidx, long long npos, const float* w, const float* ht, const float* bias,
               const float* drive, int n_s, float* out, int n_rows, int n_src, int B, void* cw, float* scratch,

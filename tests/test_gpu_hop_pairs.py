@@ -282,3 +282,31 @@ def test_a_wave_off_the_steps_boundary_is_no_wave(gpu_lib, graph, half):
     assert len(touched) and (got[touched] == 7).all()
     want[touched] = 7
     assert torch.equal(got, want)
+
+
+def test_a_re_drive_field_past_the_drive_is_none(gpu_lib, graph):
+    """fh_layer on a plan whose re-drive fields name rows past the drive, in whole and in split rows: as with -1 there
+    (the drive is the front of a larger buffer)."""
+    index, _, w, _ = graph
+    B, n_s, n_rows = 96, 50, HEAVY + LIGHT
+    h, _ = _states(B, 5)
+    drive = torch.randn(B // 32 + 1, n_s, 32, device="cuda", generator=torch.Generator(device="cuda").manual_seed(6))
+    d = dict(_plan(index[0], index[1], None, w.numel()))
+    seg, split = d["seg"].clone(), d["split"].clone()
+    seg[:, 2] = torch.where(seg[:, 0] >= 0, seg[:, 0] % (2 * n_s), -1).to(torch.int32)
+    split[:, 3] = split[:, 0] % (2 * n_s)
+
+    def layer(seg, split):
+        out = torch.full((B // 32, n_rows, 32), 7.0, device="cuda")
+        cw = torch.empty(d["npos"], 2, dtype=torch.int32, device="cuda")
+        part = torch.empty(max(d["nslot"] * B, 1), device="cuda")
+        src = tiled(h)
+        call("fh_layer", *_args(dict(d, seg=seg, split=split)), w.data_ptr(), src.data_ptr(), None, drive.data_ptr(), n_s,
+             out.data_ptr(), n_rows, N_SRC, B, cw.data_ptr(), part.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        return out
+    got = layer(seg, split)
+    seg[:, 2][seg[:, 2] >= n_s] = -1
+    split[:, 3][split[:, 3] >= n_s] = -1
+    assert torch.equal(got, layer(seg, split))
+    assert not torch.equal(got, layer(d["seg"], d["split"]))
